@@ -233,7 +233,7 @@ static void drop_tag(Buffer* b, bool park = false) {
   }
 }
 void tag_bn_stats(void* y, void* side, uint32_t B, uint32_t C, uint32_t S, uint32_t pieces,
-                  uint32_t H, uint32_t W) {
+                  uint32_t H, uint32_t W, uint32_t gLayout) {
   Buffer* Y = static_cast<Buffer*>(y);
   if (!Y || Y->magic != kMagicLive) {
     release_buffer(side);
@@ -247,6 +247,7 @@ void tag_bn_stats(void* y, void* side, uint32_t B, uint32_t C, uint32_t S, uint3
   Y->meta[3] = H;
   Y->meta[4] = W;
   Y->aux32 = pieces;
+  Y->aux32b = gLayout;
   Y->side = static_cast<Buffer*>(side);
 }
 // The activation that followed each batch norm (keyed by its gamma buffer
@@ -377,8 +378,8 @@ bool bn_act_adopt(void* z, void* a, uint32_t act, uint32_t n) {
   return true;
 }
 
-void tag_grad_g_nhwc(void* dx, void* side, uint32_t B, uint32_t C, uint32_t H, uint32_t W,
-                     uint32_t rows) {
+void tag_grad_g(void* dx, void* side, uint32_t layout, uint32_t B, uint32_t C, uint32_t H,
+                uint32_t W, uint32_t rows) {
   Buffer* D = static_cast<Buffer*>(dx);
   if (!D || D->magic != kMagicLive) {
     release_buffer(side);
@@ -386,7 +387,7 @@ void tag_grad_g_nhwc(void* dx, void* side, uint32_t B, uint32_t C, uint32_t H, u
   }
   drop_tag(D);
   set_tag(D, kGradGTag);
-  D->meta[0] = kGLayoutNhwc;
+  D->meta[0] = layout;
   D->meta[1] = B;
   D->meta[2] = C;
   D->meta[3] = H;
@@ -991,7 +992,7 @@ void* ConvForwardFused(void* x, void* filters, void* bias, uint32_t batch, uint3
     if (sreq.pieces) {
       const bool gn = conv_g_nhwc_pass(g);
       tag_bn_stats(out, sctx.side, batch, outC, g.OH * g.OW, sreq.pieces, gn ? g.OH : 0,
-                   gn ? g.OW : 0);
+                   gn ? g.OW : 0, conv_g_layout(g));
     }
     else
       release_buffer(sctx.side);
@@ -1053,7 +1054,7 @@ void ConvBackwardFused(void* gradOut, void* fwdOut, void* x, void* filters, void
       // conv with no ReLU mask.
       if ((Y && gMatch && DY->src == Y && tag_alive(Y, kReluOutTag, DY->srcGen) &&
            DY->meta[0] == conv_g_layout(g)) ||
-          (!Y && actType != 1 && gMatch && DY->meta[0] == kGLayoutNhwc && conv_g_nhwc_pass(g))) {
+          (!Y && actType != 1 && gMatch && DY->meta[0] == conv_g_layout(g) && conv_g_nhwc_pass(g))) {
         pre.layout = DY->meta[0];
         pre.g = DY->side->ptr;
         pre.db = pre.g + g_side_floats(pre.layout, batch, outC, g.OH, g.OW);

@@ -1,0 +1,290 @@
+// The input gradient GEMM of the convolutions: filters (rows c) x G patches
+// (rows = input pixels).  On bf16 parts (dce_igemm_parts.h) or, for few
+// channels, on fp32 MFMAs (dce_igemm.h).
+#include "dce_igemm_parts.h"
+
+namespace dce {
+
+template <bool S1, bool BLK>
+struct DxRun {
+  const float* wt;
+  const float* gn;
+  float* dx;
+  float* part;
+  ConvGeom g;
+  uint32_t splits;
+  template <int MT, int NT, int KT>
+  int occ(bool split) const {
+    using LA = LdDenseRK<MT, KT>;
+    using LB = LdPixRK<NT, KT, false, S1, BLK>;
+    return split ? occupancy(k_igemm<MT, NT, KT, LA, LB, EpiRowMajor>)
+                 : occupancy(k_igemm<MT, NT, KT, LA, LB, EpiNCHW>);
+  }
+  template <int MT, int NT, int KT>
+  bool run() {
+    const uint32_t OCp = pad4(g.OC), KK = g.k * g.k, kdim = KK * OCp;
+    const uint32_t HW = g.H * g.W, N = g.B * HW;
+    using LA = LdDenseRK<MT, KT>;
+    using LB = LdPixRK<NT, KT, false, S1, BLK>;
+    const typename LA::Params pa{wt, kdim, g.C, kdim, g.C * kdim};
+    const typename LB::Params pb{gn, g.OH, g.OW, OCp, g.k, g.s, g.p, g.W, HW, N, kdim,
+                                 g.B * g.OH * g.OW * OCp, make_fastdiv(HW), make_fastdiv(g.W),
+                                 make_fastdiv(BLK ? KK : OCp), make_fastdiv(g.k)};
+    const uint32_t kt = cdiv(kdim, KT);
+    const EpiNCHW::Params pe{dx, nullptr, g.C, HW, N, 0, make_fastdiv(HW)};
+    if (splits > 1) {
+      const EpiRowMajor::Params pr{part, g.C, N, N, g.C * N};
+      return launch<MT, NT, KT, LA, LB, EpiRowMajor>(pa, pb, pr, g.C, N, kt, splits,
+                                                    "conv_backward_input") &&
+             split_nchw(part, nullptr, dx, g.C, N, HW, splits, 0);
+    }
+    return launch<MT, NT, KT, LA, LB, EpiNCHW>(pa, pb, pe, g.C, N, kt, 1, "conv_backward_input");
+  }
+};
+
+// One sub-pixel phase of a strided dX (s > 1).  The input pixels (b, ph +
+// s*a, pw + s*c) receive only the taps kh = rh + s*jh (jh < nh), kw = rw +
+// s*jw (jw < nw) with rh = (ph + p) mod s, whose output pixels are (a + qh -
+// jh, c + qw - jw), qh = (ph + p - rh) / s: a stride-1 gather over the
+// phase's own GH x GW grid with an nh x nw kernel.
+struct PhaseGeom {
+  uint32_t ph, pw, rh, rw, nh, nw, qh, qw, GH, GW;
+};
+
+template <bool BLK>
+struct DxPhaseRun {
+  const float* wt;
+  const float* gn;
+  float* dx;
+  ConvGeom g;
+  PhaseGeom q;
+  template <int MT, int NT, int KT>
+  int occ(bool) const {
+    return occupancy(
+        k_igemm<MT, NT, KT, LdDenseRK<MT, KT>, LdPixRK<NT, KT, false, true, BLK>, EpiNCHWPhase>);
+  }
+  template <int MT, int NT, int KT>
+  bool run() {
+    const uint32_t OCp = pad4(g.OC), KK = q.nh * q.nw, kdim = KK * OCp;
+    const uint32_t GHW = q.GH * q.GW, N = g.B * GHW;
+    using LA = LdDenseRK<MT, KT>;
+    using LB = LdPixRK<NT, KT, false, true, BLK>;
+    const typename LA::Params pa{wt, kdim, g.C, kdim, g.C * kdim};
+    const typename LB::Params pb{gn, g.OH, g.OW, OCp, q.nw, 1, q.qh, q.GW, GHW, N, kdim,
+                                 g.B * g.OH * g.OW * OCp, make_fastdiv(GHW), make_fastdiv(q.GW),
+                                 make_fastdiv(BLK ? KK : OCp), make_fastdiv(q.nw),
+                                 int(q.qw) - int(q.qh)};
+    const EpiNCHWPhase::Params pe{dx, g.C, g.H, g.W, q.GW, GHW, N, g.s, q.ph, q.pw,
+                                  make_fastdiv(GHW), make_fastdiv(q.GW)};
+    return launch<MT, NT, KT, LA, LB, EpiNCHWPhase>(pa, pb, pe, g.C, N, cdiv(kdim, KT), 1,
+                                                    "conv_backward_input");
+  }
+};
+
+// dX on parts: the whole gather (the phase fields unused), or one phase.
+template <bool S1, class EPI>
+struct DxPartsRun {
+  const float* wt;
+  const float* gn;
+  float* dx;
+  float* part;
+  ConvGeom g;
+  uint32_t splits;
+  PhaseGeom q;
+  static constexpr bool PHASE = std::is_same<EPI, PEpiPhase>::value;
+  template <int MT, int NT>
+  int occ(bool split) const {
+    return split ? occupancy(k_gemm_parts<MT, NT, PRows<MT>, PPix<NT, S1>, PEpiRowMajor>)
+                 : occupancy(k_gemm_parts<MT, NT, PRows<MT>, PPix<NT, S1>, EPI>);
+  }
+  template <int MT, int NT>
+  bool run() const {
+    const uint32_t no = pad16(g.OC) / 16, KK = PHASE ? q.nh * q.nw : g.k * g.k, kt = KK * no;
+    const uint32_t GW = PHASE ? q.GW : g.W, GHW = PHASE ? q.GH * q.GW : g.H * g.W, N = g.B * GHW;
+    const uint32_t kw = PHASE ? q.nw : g.k;
+    const char* what = "conv_backward_input";
+    using LA = PRows<MT>;
+    using LB = PPix<NT, S1>;
+    const typename LA::Params pa{wt, g.C, kt, g.C * kt * 24};
+    const typename LB::Params pb{gn, g.OH, g.OW, no, kw, PHASE ? 1 : g.s, PHASE ? q.qh : g.p, GW, GHW,
+                                 N, uint32_t(parts_floats(size_t(g.B) * g.OH * g.OW, g.OC)),
+                                 make_fastdiv(GHW), make_fastdiv(GW), make_fastdiv(KK),
+                                 make_fastdiv(kw), PHASE ? int(q.qw) - int(q.qh) : 0};
+    if constexpr (PHASE) {
+      const EpiNCHWPhase::Params pe{dx, g.C, g.H, g.W, GW, GHW, N, g.s, q.ph, q.pw, pb.dGridHW,
+                                    pb.dGridW};
+      return launch_parts<MT, NT, LA, LB, PEpiPhase>(pa, pb, pe, g.C, N, kt, 1, what);
+    } else {
+      if (splits > 1) {
+        const EpiRowMajor::Params pr{part, g.C, N, N, g.C * N};
+        return launch_parts<MT, NT, LA, LB, PEpiRowMajor>(pa, pb, pr, g.C, N, kt, splits, what) &&
+               split_nchw(part, nullptr, dx, g.C, N, GHW, splits, 0);
+      }
+      const EpiNCHW::Params pe{dx, nullptr, g.C, GHW, N, 0, pb.dGridHW};
+      return launch_parts<MT, NT, LA, LB, PEpiNCHW>(pa, pb, pe, g.C, N, kt, 1, what);
+    }
+  }
+};
+
+// The four phases of a stride-2 dX on parts in one launch, their filters
+// re-laid by another; phases that no tap reaches (k = 1) are zero.
+struct DxMulti {
+  using EPI = PEpiPhase;
+  const float* gn;
+  float* dx;
+  ConvGeom g;
+  PhaseGeom q[4];
+  const float* wt[4];
+  uint32_t n;
+  template <int MT, int NT>
+  int occ(bool) const {
+    return occupancy(k_gemm_parts_multi<MT, NT, PRows<MT>, PPix<NT, true>, EPI>);
+  }
+  template <int MT, int NT>
+  bool run() const {
+    PMulti<PRows<MT>, PPix<NT, true>, EPI> a{};
+    const uint32_t no = pad16(g.OC) / 16;
+    a.gm = cdiv(g.C, MT);
+    uint32_t wgs = 0;
+    for (uint32_t i = 0; i < 4; ++i) {
+      a.first[i] = i < n ? wgs : 0xFFFFFFFFu;
+      if (i >= n) continue;
+      const PhaseGeom& f = q[i];
+      const uint32_t KK = f.nh * f.nw, GHW = f.GH * f.GW, N = g.B * GHW;
+      a.ktiles[i] = KK * no;
+      a.pa[i] = {wt[i], g.C, KK * no, g.C * KK * no * 24};
+      a.pb[i] = {gn, g.OH, g.OW, no, f.nw, 1, f.qh, f.GW, GHW, N,
+                 uint32_t(parts_floats(size_t(g.B) * g.OH * g.OW, g.OC)), make_fastdiv(GHW),
+                 make_fastdiv(f.GW), make_fastdiv(KK), make_fastdiv(f.nw), int(f.qw) - int(f.qh)};
+      a.pe[i] = {dx, g.C, g.H, g.W, f.GW, GHW, N, g.s, f.ph, f.pw, a.pb[i].dGridHW, a.pb[i].dGridW};
+      wgs += a.gm * cdiv(N, NT);
+    }
+    hipLaunchKernelGGL((k_gemm_parts_multi<MT, NT, PRows<MT>, PPix<NT, true>, EPI>), dim3(wgs),
+                       dim3(kThreads), 0, stream(), a);
+    return check_launch("conv_backward_input");
+  }
+};
+template <class Geom>
+static bool phases_in_one(const float* w, float* wt, const float* gn, float* dx, const ConvGeom& g,
+                          Geom&& geom) {
+  const uint32_t OCp = pad16(g.OC);
+  DxMulti m{};
+  m.gn = gn;
+  m.dx = dx;
+  m.g = g;
+  WPerm4 pw{};
+  uint32_t cols = 0, kmax = 0;
+  bool empty = false;
+  float* at = wt;
+  for (uint32_t i = 0; i < 4; ++i) {
+    const PhaseGeom q = geom(i / 2, i % 2);
+    const uint32_t KK = q.nh * q.nw;
+    if (q.GH * q.GW == 0) continue;
+    if (KK == 0) {
+      empty = true;
+      continue;
+    }
+    pw.p[m.n] = WPerm{w, at, g.OC, g.C, KK, OCp, KK * OCp, 1, 1, q.nw, g.k, 2, q.rh, q.rw, 1u};
+    m.wt[m.n] = at;
+    m.q[m.n++] = q;
+    at += parts_floats(size_t(g.C) * KK, g.OC);
+    cols += g.B * q.GH * q.GW;
+    kmax = std::max(kmax, KK * OCp);
+  }
+  if (empty && !fill_zero(dx, size_t(g.B) * g.C * g.H * g.W)) return false;
+  if (m.n == 0) return true;
+  if (!permute_w4(pw)) return false;
+  const TileCfg t = parts_choose("DCE_TUNE_DX", g.C, cols, kmax, 1, true,
+                                 [&](const TileCfg& v) { return parts_occ(v, m); });
+  return parts_dispatch(t, m);
+}
+
+// dX of a strided convolution as its s*s sub-pixel phases: every input pixel
+// multiplies only the taps that reach it, where the strided gather walks all
+// k*k taps for every pixel and finds all but about 1/s^2 of them out of
+// step.  Each phase gets its own filter re-layout (into wt, C * k*k * OCp
+// floats) and GEMM, unsplit; phases that no tap reaches (k < s) are zero.
+bool conv_dx_phased(const float* w, float* wt, const float* gn, float* dx, const ConvGeom& g,
+                    bool parts) {
+  const uint32_t s = g.s, OCp = parts ? pad16(g.OC) : pad4(g.OC);
+  const bool blk = blocked_k(OCp);
+  auto geom = [&](uint32_t ph, uint32_t pw) {
+    PhaseGeom q{};
+    q.ph = ph;
+    q.pw = pw;
+    q.GH = ph < g.H ? cdiv(g.H - ph, s) : 0;
+    q.GW = pw < g.W ? cdiv(g.W - pw, s) : 0;
+    q.rh = (ph + g.p) % s;
+    q.rw = (pw + g.p) % s;
+    q.nh = q.rh < g.k ? cdiv(g.k - q.rh, s) : 0;
+    q.nw = q.rw < g.k ? cdiv(g.k - q.rw, s) : 0;
+    q.qh = (ph + g.p - q.rh) / s;
+    q.qw = (pw + g.p - q.rw) / s;
+    return q;
+  };
+  if (parts && s == 2) return phases_in_one(w, wt, gn, dx, g, geom);
+  bool empty = false;
+  for (uint32_t ph = 0; ph < s; ++ph)
+    for (uint32_t pw = 0; pw < s; ++pw) {
+      const PhaseGeom q = geom(ph, pw);
+      empty |= q.GH * q.GW > 0 && q.nh * q.nw == 0;
+    }
+  if (empty && !fill_zero(dx, size_t(g.B) * g.C * g.H * g.W)) return false;
+  for (uint32_t ph = 0; ph < s; ++ph)
+    for (uint32_t pw = 0; pw < s; ++pw) {
+      const PhaseGeom q = geom(ph, pw);
+      if (q.GH * q.GW == 0 || q.nh * q.nw == 0) continue;
+      const uint32_t KK = q.nh * q.nw, kdim = KK * OCp, N = g.B * q.GH * q.GW;
+      if (!permute_w(WPerm{w, wt, g.OC, g.C, KK, OCp, kdim, 1, blk ? 1 : 0, q.nw, g.k, s, q.rh,
+                           q.rw, parts ? 1u : 0u}))
+        return false;
+      if (parts) {
+        const DxPartsRun<true, PEpiPhase> run{wt, gn, dx, nullptr, g, 1, q};
+        const TileCfg t = parts_choose("DCE_TUNE_DX", g.C, N, kdim, 1, true,
+                                       [&](const TileCfg& v) { return parts_occ(v, run); });
+        if (!parts_dispatch(t, run)) return false;
+        continue;
+      }
+      TileCfg c = choose(
+          "DCE_TUNE_DX", g.C, N, kdim, 1, true,
+          [&](const TileCfg& t) {
+            return blk ? tiles_occ16(t, DxPhaseRun<true>{}) : tiles_occ16(t, DxPhaseRun<false>{});
+          },
+          true);
+      narrow_short_k(c, "DCE_TUNE_DX", g.C, N, kdim);
+      c.splits = 1;
+      const bool ok = blk ? tiles_dispatch16(c, DxPhaseRun<true>{wt, gn, dx, g, q})
+                          : tiles_dispatch16(c, DxPhaseRun<false>{wt, gn, dx, g, q});
+      if (!ok) return false;
+    }
+  return true;
+}
+
+
+TileCfg conv_dx_choose(const ConvGeom& g, bool parts) {
+  const uint32_t N = g.B * g.H * g.W;
+  const bool s1 = g.s == 1;
+  if (parts)
+    return parts_choose("DCE_TUNE_DX", g.C, N, g.k * g.k * pad16(g.OC), 8, true,
+                        [&](const TileCfg& t) {
+                          return s1 ? parts_occ(t, DxPartsRun<true, PEpiNCHW>{})
+                                    : parts_occ(t, DxPartsRun<false, PEpiNCHW>{});
+                        });
+  const uint32_t OCp = pad4(g.OC), kdim = g.k * g.k * OCp;
+  const bool blk = blocked_k(OCp);
+  TileCfg c = choose(
+      "DCE_TUNE_DX", g.C, N, kdim, 8, true,
+      [&](const TileCfg& t) { return conv_variant_occ<DxRun>(s1, blk, t); }, true);
+  narrow_short_k(c, "DCE_TUNE_DX", g.C, N, kdim);
+  return c;
+}
+bool conv_dx_gemm(const TileCfg& c, const float* wt, const float* gn, float* dx, float* part,
+                  const ConvGeom& g, bool parts) {
+  if (parts)
+    return g.s == 1
+               ? parts_dispatch(c, DxPartsRun<true, PEpiNCHW>{wt, gn, dx, part, g, c.splits, {}})
+               : parts_dispatch(c, DxPartsRun<false, PEpiNCHW>{wt, gn, dx, part, g, c.splits, {}});
+  return conv_variant<DxRun>(g.s == 1, blocked_k(pad4(g.OC)), c, wt, gn, dx, part, g, c.splits);
+}
+
+}  // namespace dce

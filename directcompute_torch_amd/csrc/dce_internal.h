@@ -39,7 +39,8 @@ struct Buffer {
   //            the per-channel double sums of y and y*y as [C][pieces][2],
   //            meta = {B, C, H*W, H, W}, aux32 = pieces; meta[3..4] are 0
   //            unless the conv's backward reads its gradient as an NHWC G
-  //            (then batchnorm_backward_dx over y makes that G);
+  //            (then batchnorm_backward_dx over y makes that G, in the layout
+  //            aux32b);
   //  kGradGTag also marks the dx of batchnorm_backward_dx over such a y:
   //            side = [NHWC G | bias-gradient partials], src = null;
   //  kBnOutTag: output z of batchnorm_forward; key = that call's gamma
@@ -85,12 +86,15 @@ constexpr uint32_t kBnGradPartTag = 0x9009u;
 // Layouts of a conv backward's masked gradient G.
 constexpr uint32_t kGLayoutPad = 1;   // [B*OC][OH][pad4(OW)], zero past OW (stride-phase dW)
 constexpr uint32_t kGLayoutNhwc = 2;  // [B*OH*OW][pad4(OC)] (the transpose pass)
+constexpr uint32_t kGLayoutParts = 3; // [B*OH*OW][pad16(OC)] as bf16 parts (the transpose pass)
 
 // Floats of G in `layout` for a conv output [B][C][H][W], rounded up to 64
 // (the bias-gradient partials follow it in a kGradGTag side buffer).
 inline size_t g_side_floats(uint32_t layout, uint32_t B, uint32_t C, uint32_t H, uint32_t W) {
-  const size_t n = layout == kGLayoutNhwc ? size_t(B) * H * W * ((C + 3u) & ~3u)
-                                          : size_t(B) * C * H * ((W + 3u) & ~3u);
+  const size_t pix = size_t(B) * H * W;
+  const size_t n = layout == kGLayoutNhwc    ? pix * ((C + 3u) & ~3u)
+                   : layout == kGLayoutParts ? pix * ((C + 15u) / 16) * 24
+                                             : size_t(B) * C * H * ((W + 3u) & ~3u);
   return (n + 63) & ~size_t(63);
 }
 
@@ -139,7 +143,7 @@ void release_buffer(void* h);
 // on) holds the per-channel double sums of y and y*y, [C][pieces][2].  H, W:
 // the plane of a conv output whose backward reads an NHWC G (else 0, 0).
 void tag_bn_stats(void* y, void* side, uint32_t B, uint32_t C, uint32_t S, uint32_t pieces,
-                  uint32_t H = 0, uint32_t W = 0);
+                  uint32_t H = 0, uint32_t W = 0, uint32_t gLayout = 0);
 // The activation (1 relu, 2 relu6, 0 none seen) that last followed the batch
 // norm whose gamma buffer is `gamma`.
 uint32_t bn_act_guess(const void* gamma);
@@ -174,8 +178,8 @@ const double* bn_grad_part_of(void* dy, void* x, void* mean, void* var, uint32_t
 bool bn_act_adopt(void* z, void* a, uint32_t act, uint32_t n);
 // Tag dx kGradGTag with an NHWC G side buffer (owned by dx from now on) for
 // the conv whose output has B x C channels of H x W; rows = db partial rows.
-void tag_grad_g_nhwc(void* dx, void* side, uint32_t B, uint32_t C, uint32_t H, uint32_t W,
-                     uint32_t rows);
+void tag_grad_g(void* dx, void* side, uint32_t layout, uint32_t B, uint32_t C, uint32_t H,
+                uint32_t W, uint32_t rows);
 
 // ---------------------------------------------------------------------------
 // Fast unsigned division by a run-time constant (numerators < 2^31).
@@ -231,6 +235,11 @@ struct BRes {
   __device__ __forceinline__ void ld4_lds(uint32_t off, float* lds) const {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         r, (__attribute__((address_space(3))) void*)lds, 16, off * 4u, 0, 0, 0);
+  }
+  // The same from a byte offset.
+  __device__ __forceinline__ void ld16_lds(uint32_t bytes, char* lds) const {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        r, (__attribute__((address_space(3))) void*)lds, 16, bytes, 0, 0, 0);
   }
 };
 
@@ -449,26 +458,26 @@ struct ConvStatsReq {
 // the copy of x (xcopy_floats(g) floats) for a later backward.
 bool conv_forward(const float* x, float* x_nhwc_keep, const float* w, const float* bias,
                   float* y, const ConvGeom& g, uint32_t act, ConvStatsReq* st = nullptr);
-// The layout of G that conv_backward reads for this geometry (kGLayoutPad or
-// kGLayoutNhwc), and the padded row width of kGLayoutPad.
+// The layout of G that conv_backward reads for this geometry, and the padded
+// row width of kGLayoutPad.
 uint32_t conv_g_layout(const ConvGeom& g);
 // Does the backward of this conv without a ReLU mask make an NHWC G (the
 // transpose pass)?  Not for pointwise or fewer-than-4-channel layers.
 bool conv_g_nhwc_pass(const ConvGeom& g);
 // batchnorm_backward_dx (x, dy, the statistics and gamma, dgamma, dbeta of C
-// channels over B planes of HW) writing dx and, with it, the NHWC G of dx
-// (dx transposed to [B*HW][pad4(C)]) and the bias-gradient partials that a
-// conv backward's transpose pass would make: g_side_floats(kGLayoutNhwc, ...)
+// channels over B planes of HW) writing dx and, with it, the G of dx (dx
+// transposed, as fp32 or bf16 parts by `layout`) and the bias-gradient partials that a
+// conv backward's transpose pass would make: g_side_floats(layout, ...)
 // floats of G, then C x rows partials.  rows = bn_dx_g_rows(B, C, HW).
 uint32_t bn_dx_g_rows(uint32_t B, uint32_t C, uint32_t HW);
 bool bn_dx_g(const float* x, const float* dy, const float* mean, const float* var,
              const float* gamma, const float* dg, const float* db, float eps, float* dx,
-             float* g, float* dbPart, uint32_t B, uint32_t C, uint32_t HW);
+             uint32_t layout, float* g, float* dbPart, uint32_t B, uint32_t C, uint32_t HW);
 uint32_t conv_g_pad_width(const ConvGeom& g);
 // A masked gradient G made by the producer of dy (the max-pool backward):
 // g in `layout` (kGLayoutPad), db = bias-gradient partials [OC][dbRows].
 struct PreG {
-  uint32_t layout;  // kGLayoutPad (a ReLU conv's masked G) or kGLayoutNhwc (no mask)
+  uint32_t layout;  // kGLayoutPad (a ReLU conv's masked G), or kGLayoutNhwc / kGLayoutParts (no mask)
   const float* g;
   const float* db;
   uint32_t dbRows;

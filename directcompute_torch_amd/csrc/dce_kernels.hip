@@ -1091,7 +1091,7 @@ static bool bn_elem(const char* what, const Dispatch& d) {
   return check_launch(what);
 }
 static bool sh_bn_forward(const Dispatch& d) { return bn_elem<0>("batchnorm_forward", d); }
-// Over the output of a conv whose backward reads an NHWC G (the forward's
+// Over the output of a conv whose backward reads a transposed G (the forward's
 // tag says so), dx comes with that G and its bias-gradient partials (owned
 // by dx, kGradGTag), and the conv backward then runs no transpose pass.
 static bool sh_bn_backward_dx(const Dispatch& d) {
@@ -1104,7 +1104,8 @@ static bool sh_bn_backward_dx(const Dispatch& d) {
     const uint64_t total = uint64_t(N) * C * Sz;
     const Buf x = S(d, 0), dy = S(d, 1), mean = S(d, 2), var = S(d, 3), gamma = S(d, 4),
               dg = S(d, 5), db = S(d, 6), out = U(d, 0);
-    const size_t nG = g_side_floats(kGLayoutNhwc, N, C, X->meta[3], X->meta[4]);
+    const uint32_t layout = X->aux32b;
+    const size_t nG = g_side_floats(layout, N, C, X->meta[3], X->meta[4]);
     const uint32_t rows = bn_dx_g_rows(N, C, Sz);
     const uint64_t side_n = nG + uint64_t(rows) * C;
     if (covers(x, total) && covers(dy, total) && covers(out, total) && covers(mean, C) &&
@@ -1112,12 +1113,12 @@ static bool sh_bn_backward_dx(const Dispatch& d) {
         side_n < 0xFFFFFFFFull) {
       Buffer* side = static_cast<Buffer*>(create_buffer(nullptr, uint32_t(side_n)));
       if (side) {
-        if (!bn_dx_g(x.p, dy.p, mean.p, var.p, gamma.p, dg.p, db.p, eps, out.p, side->ptr,
-                     side->ptr + nG, N, C, Sz)) {
+        if (!bn_dx_g(x.p, dy.p, mean.p, var.p, gamma.p, dg.p, db.p, eps, out.p, layout,
+                     side->ptr, side->ptr + nG, N, C, Sz)) {
           release_buffer(side);
           return false;
         }
-        tag_grad_g_nhwc(d.uavs[0], side, N, C, X->meta[3], X->meta[4], rows);
+        tag_grad_g(d.uavs[0], side, layout, N, C, X->meta[3], X->meta[4], rows);
         return true;
       }
     }

@@ -1,0 +1,140 @@
+"""Conv backward on bf16 parts (dW and dX as six bf16 MFMA products per fp32
+product) against the float64 oracle: tile edges, channels that fill no block of
+16, strides with their sub-pixel phases, split-K, and operands that are
+infinite, NaN, overflowing or tiny.
+
+Bound per element, from the arithmetic: with S the same sum over |a||b| and n
+steps of 16 k, the dropped part products are below 2^-21 S each, and a step
+rounds the accumulator twice and its inner sum once per product group (6 at
+most), all below 2^-24 of a partial sum that S bounds; split-K adds one rounding
+per split (at most 256) of the partial sums."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import kernels as K
+from tests.helpers import download, he, release, rng, upload
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # B, C, H, W, OC, k, s, p, act
+    (2, 64, 9, 7, 64, 3, 1, 1, 0),        # one 64-row tile, ragged pixels
+    (2, 65, 8, 8, 64, 3, 1, 1, 1),        # one channel past a tile and a block
+    (1, 48, 11, 13, 128, 3, 1, 1, 1),
+    (3, 37, 13, 9, 70, 5, 1, 2, 0),       # channels padded to 48 and 80
+    (2, 33, 7, 7, 129, 3, 1, 0, 1),       # no padding; 129 output rows
+    (1, 32, 6, 6, 384, 5, 1, 2, 0),       # few rows, long K
+    (2, 128, 5, 5, 130, 3, 1, 1, 0),
+    (4, 96, 32, 32, 64, 3, 1, 1, 1),      # split-K dW
+    (2, 64, 12, 10, 96, 3, 2, 1, 1),      # stride 2: four phases in one launch
+    (2, 40, 13, 11, 70, 5, 2, 2, 0),      # odd image, phases of unequal size
+    (1, 64, 1, 9, 64, 3, 2, 1, 0),        # phases with no rows
+    (2, 512, 8, 8, 480, 1, 2, 0, 0),      # k < s: three phases no tap reaches
+    (2, 64, 14, 14, 64, 4, 3, 1, 1),      # stride 3: one launch per phase
+    (2, 512, 6, 6, 480, 1, 1, 0, 1),      # pointwise with a ReLU mask
+]
+
+
+def _backward(eng, x, w, dy, y, s, p, act, pim=None):
+    B, C, H, W = x.shape
+    OC, _, k, _ = w.shape
+    hs = [upload(eng, a) for a in (dy, x, w)]
+    hy = upload(eng, y) if act == 1 else None
+    pdf, pdb, pdx = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    eng.lib.ConvBackwardFused(hs[0], hy, hs[1], hs[2], pim, B, C, H, W, OC, k, k, s, p, act, 1, 1, 1,
+                              ctypes.byref(pdf), ctypes.byref(pdb), ctypes.byref(pdx))
+    assert pdf.value and pdb.value and pdx.value, eng.last_error()
+    out = (download(eng, pdf.value, w.shape), download(eng, pdb.value, (OC,)), download(eng, pdx.value, x.shape))
+    release(eng, *hs, hy, pdf.value, pdb.value, pdx.value)
+    return out
+
+
+def _inputs(B, C, H, W, OC, k, s, p, act):
+    r = rng(77 + B + 3 * C + 5 * H + 7 * OC + 11 * k + s)
+    x = r.standard_normal((B, C, H, W)).astype(np.float32)
+    w = he(r, (OC, C, k, k), C * k * k)
+    OH, OW = K.conv_out_hw(H, W, k, s, p)
+    dy = r.standard_normal((B, OC, OH, OW)).astype(np.float32)
+    y = r.standard_normal(dy.shape).astype(np.float32)
+    return x, w, dy, y
+
+
+def _check(got, x, w, dy, y, s, p, act):
+    OC, C, k, _ = w.shape
+    ref = K.conv_backward(dy, y, x, w, s, p, act)
+    S = K.conv_backward(np.abs(dy), y, np.abs(x), np.abs(w), s, p, act)
+    for name, a, b, t, n in (("dW", got[0], ref[0], S[0], dy.size // OC), ("dX", got[2], ref[2], S[2], OC * k * k)):
+        bound = (3 * 2.0 ** -21 + (8 * (n / 16 + 2) + 256) * 2.0 ** -24) * t + 1e-37
+        worst = np.max(np.abs(a - b) - bound)
+        assert worst <= 0, f"{name}: {worst:.3e} past the bound"
+    # db: fp32 sums of at most B*OH*OW values
+    assert np.all(np.abs(got[1] - ref[1]) <= (dy.size // OC) * 2.0 ** -24 * S[1] + 1e-37)
+
+
+@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("keep", [True, False])
+def test_backward_on_parts(eng, case, keep):
+    """With the copy of x that the forward keeps, and rebuilt from x."""
+    B, C, H, W, OC, k, s, p, act = case
+    x, w, dy, y = _inputs(*case)
+    pim = ctypes.c_void_p()
+    if keep:
+        hx, hw, hb = upload(eng, x), upload(eng, w), upload(eng, np.zeros(OC, np.float32))
+        hy = eng.lib.ConvForwardFused(hx, hw, hb, B, C, H, W, OC, k, k, s, p, 0, ctypes.byref(pim))
+        assert hy, eng.last_error()
+        yref = K.conv_forward(x, w, np.zeros(OC, np.float32), s, p, 0)
+        assert np.max(np.abs(download(eng, hy, yref.shape) - yref)) <= 1e-4 * np.max(np.abs(yref))
+        release(eng, hx, hw, hb, hy)
+    _check(_backward(eng, x, w, dy, y, s, p, act, pim.value), x, w, dy, y, s, p, act)
+
+
+@pytest.mark.parametrize("tile", ["128,128,16,1", "128,64,16,3", "64,128,16,2", "64,64,16,5"])
+def test_forced_tiles(eng, monkeypatch, tile):
+    monkeypatch.setenv("DCE_TUNE_DW", tile)
+    monkeypatch.setenv("DCE_TUNE_DX", tile)
+    for case in (CASES[3], CASES[4], CASES[7]):
+        x, w, dy, y = _inputs(*case)
+        s, p, act = case[6:]
+        _check(_backward(eng, x, w, dy, y, s, p, act), x, w, dy, y, s, p, act)
+
+
+@pytest.mark.parametrize("what", ["inf", "nan", "quiet", "overflow", "tiny"])
+def test_special_values(eng, what):
+    """Infinities and NaNs come out where IEEE arithmetic puts them (the tile is
+    computed again in fp32), and values whose last part leaves the bf16 range
+    lose no more than that."""
+    case = (2, 64, 9, 10, 80, 3, 1, 1, 0)
+    x, w, dy, y = _inputs(*case)
+    s, p, act = case[6:]
+    if what == "inf":
+        dy[0, 5, 4, 4], x[1, 7, 3, 3] = np.inf, -np.inf
+    elif what == "nan":
+        dy[1, 60, 0, 0] = np.nan
+    elif what == "quiet":  # a NaN whose payload sits in the low 16 bits alone
+        dy[1, 60, 0, 0] = np.array([0x7F800001], np.uint32).view(np.float32)[0]
+    elif what == "overflow":
+        dy[0, 3, 2, 2], w[3, :, :, :] = 3e38, 3e5
+    else:
+        dy *= np.float32(1e-36)
+    with np.errstate(all="ignore"):
+        ref = K.conv_backward(dy, y, x, w, s, p, act)
+    got = _backward(eng, x, w, dy, y, s, p, act)
+    for a, b in ((got[0], ref[0]), (got[2], ref[2])):
+        with np.errstate(all="ignore"):
+            b32 = b.astype(np.float32)
+        assert np.array_equal(np.isnan(a), np.isnan(b32))
+        assert np.array_equal(np.isinf(a), np.isinf(b32))
+        inf = np.isinf(b32)
+        assert np.array_equal(a[inf], b32[inf])
+        fin = np.isfinite(b32)
+        scale = np.max(np.abs(b[fin])) if what != "overflow" else np.maximum(np.abs(b[fin]), 1.0)
+        # tiny: operands of 1e-36 keep 16 bits (2^-15 of an operand at worst)
+        tol = 2.0 ** -14 if what == "tiny" else 1e-5
+        if what == "overflow":  # sums of huge terms cancel: relative to the sum of magnitudes
+            Sm = K.conv_backward(np.abs(dy), y, np.abs(x), np.abs(w), s, p, act)
+            Sm = (Sm[0] if a is got[0] else Sm[2])[fin]
+            assert np.all(np.abs(a[fin] - b[fin]) <= 1e-5 * Sm + 1e-30)
+        else:
+            assert np.max(np.abs(a[fin] - b[fin])) <= tol * scale
