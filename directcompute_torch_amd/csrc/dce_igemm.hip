@@ -899,7 +899,8 @@ bool conv_parts(const ConvGeom& g) {
   if (g.C < 32 || g.OC < 32) return false;
   if (double(g.k) * g.k * g.C * g.OC < 210.0 * (g.C + g.OC)) return false;
   return parts_floats(size_t(g.B) * g.H * g.W, g.C) < kOob &&
-         parts_floats(size_t(g.B) * g.OH * g.OW, g.OC) < kOob;
+         parts_floats(size_t(g.B) * g.OH * g.OW, g.OC) < kOob &&
+         parts_floats(size_t(g.C) * g.k * g.k, g.OC) < kOob;
 }
 
 PsGeom ps_geom(const ConvGeom& g) {
