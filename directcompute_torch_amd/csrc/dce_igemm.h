@@ -1761,6 +1761,52 @@ static inline size_t al64(size_t n) { return (n + 63) & ~size_t(63); }
 inline uint32_t pad16(uint32_t c) { return (c + 15u) & ~15u; }
 // Floats of a [rows][pad16(c)] array of bf16 parts (96 bytes per 16 values).
 inline size_t parts_floats(size_t rows, uint32_t c) { return rows * (pad16(c) / 16) * 24; }
+// x as bf16 parts (dce_igemm_parts.h), each in the upper half of a word.  An
+// infinity or a NaN (made quiet, so that its upper half is one) has no m, l.
+struct Parts {
+  uint32_t h, m, l;
+};
+__device__ __forceinline__ Parts split_parts(float x) {
+  uint32_t u = __float_as_uint(x);
+  if (x != x) u |= 0x00400000u;
+  const uint32_t hu = u & 0xffff0000u;
+  const bool fin = (u & 0x7f800000u) != 0x7f800000u;
+  const float r = x - __uint_as_float(hu);
+  const uint32_t mu = fin ? __float_as_uint(r) : 0u;
+  const float s = r - __uint_as_float(mu & 0xffff0000u);
+  return Parts{u, mu, fin ? __float_as_uint(s) : 0u};
+}
+
+// For finite x alone (4 instead of 12 instructions); others get a NaN as m.
+__device__ __forceinline__ Parts split_finite(float x) {
+  const uint32_t u = __float_as_uint(x);
+  const float r = x - __uint_as_float(u & 0xffff0000u);
+  const uint32_t mu = __float_as_uint(r);
+  return Parts{u, mu, __float_as_uint(r - __uint_as_float(mu & 0xffff0000u))};
+}
+// Parts of 8 values as one 16-byte quad per part.
+template <bool FINITE>
+__device__ __forceinline__ void split_parts8(const float (&x)[8], uint4 (&out)[3]) {
+  uint32_t h[8], m[8], l[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const Parts q = FINITE ? split_finite(x[e]) : split_parts(x[e]);
+    h[e] = q.h;
+    m[e] = q.m;
+    l[e] = q.l;
+  }
+  auto pack = [](const uint32_t (&u)[8]) {
+    uint4 v;
+    v.x = __builtin_amdgcn_perm(u[1], u[0], 0x07060302u);
+    v.y = __builtin_amdgcn_perm(u[3], u[2], 0x07060302u);
+    v.z = __builtin_amdgcn_perm(u[5], u[4], 0x07060302u);
+    v.w = __builtin_amdgcn_perm(u[7], u[6], 0x07060302u);
+    return v;
+  };
+  out[0] = pack(h);
+  out[1] = pack(m);
+  out[2] = pack(l);
+}
 bool permute_w(const WPerm& pw);
 // Four filter re-layouts in one launch (null w: none).
 struct WPerm4 {

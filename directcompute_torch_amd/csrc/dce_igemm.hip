@@ -10,22 +10,6 @@ namespace dce {
 // Side kernels: NHWC transpose (+ ReLU mask + bias-gradient partials),
 // filter re-layouts, split-K sums.
 // ---------------------------------------------------------------------------
-// x as bf16 parts (dce_igemm_parts.h), each in the upper half of a word.  An
-// infinity or a NaN (made quiet, so that its upper half is one) has no m, l.
-struct Parts {
-  uint32_t h, m, l;
-};
-__device__ __forceinline__ Parts split_parts(float x) {
-  uint32_t u = __float_as_uint(x);
-  if (x != x) u |= 0x00400000u;
-  const uint32_t hu = u & 0xffff0000u;
-  const bool fin = (u & 0x7f800000u) != 0x7f800000u;
-  const float r = x - __uint_as_float(hu);
-  const uint32_t mu = fin ? __float_as_uint(r) : 0u;
-  const float s = r - __uint_as_float(mu & 0xffff0000u);
-  return Parts{u, mu, fin ? __float_as_uint(s) : 0u};
-}
-
 __device__ __forceinline__ void permute_w_elem(const WPerm& pw, uint32_t i) {
   const float* __restrict__ w = pw.w;
   float* __restrict__ out = pw.out;

@@ -1,5 +1,6 @@
-// The flagged dense GEMM of MatMulAlloc (implicit GEMM of dce_igemm.h).
-#include "dce_igemm.h"
+// The flagged dense GEMM of MatMulAlloc: on fp32 MFMAs (dce_igemm.h),
+// large A B^T products on bf16 parts (dce_igemm_parts.h).
+#include "dce_igemm_parts.h"
 
 namespace dce {
 
@@ -37,6 +38,187 @@ struct GemmRun {
   }
 };
 
+// --------------------------------------------------------- A B^T on bf16 parts
+// The input gradient of a linear layer, dX = dY W^T.  Large ones are bound by
+// the fp32 MFMAs, at twice the time that reading W takes; as in the
+// convolutions' backward, six bf16 products stand for one fp32 product.  W is
+// read once by each row of tiles, so both operands are split on their way from
+// registers into LDS.  128 x 4096 x 9216: 97 -> 73 us; 512 x 4096 x 9216: 361 -> 281 us;
+// error against float64 4.4e-7 -> 1.9e-7 and 6.6e-7 -> 2.5e-7.
+//
+// Not taken for A^T B (the filter gradient: both operands split by a pass
+// 107 -> 106 us at 9216 x 128 x 4096, 46 -> 56 us at 4096 x 128 x 4096; its
+// eight steps of 16 do not cover the loads and the store) nor for A B (the
+// forward: 96 -> 83 us at 128 x 9216 x 4096, but another rounding there turns
+// ReLU decisions).
+
+// Rows [rows][kd] of an fp32 matrix, split between registers and stage; a
+// thread takes 8 values of one row.  kd is a multiple of 4, the base is
+// 16-byte aligned.
+template <int R>
+struct DSplit {
+  using St = PStage<R, false>;
+  struct Params {
+    const float* p;
+    uint32_t rows, kd, n;
+  };
+  struct Regs {
+    f4 v[2];
+  };
+  static_assert(2 * R <= kThreads, "at most one group of 8 per thread");
+  BRes b;
+  uint32_t base, kd, k0;
+  int slot;  // of the h part; -1: none
+  __device__ __forceinline__ void init(const Params& P, uint32_t row0, int t) {
+    b.init(P.p, P.n);
+    kd = P.kd;
+    const int row = t / 2, half = t & 1;
+    k0 = 8 * half;
+    base = row < R && row0 + row < P.rows ? (row0 + row) * P.kd + k0 : kOob;
+    slot = row < R ? row * 6 + (half ^ St::rhalf(row)) : -1;
+  }
+  __device__ __forceinline__ void load(uint32_t kt, uint32_t ke, Regs& r) const {
+    const uint32_t k = kt * 16 + k0, o = base + kt * 16;
+    const bool ok = kt < ke && base != kOob;
+    r.v[0] = b.ld4(ok && k < kd ? o : kOob);
+    r.v[1] = b.ld4(ok && k + 4 < kd ? o + 4 : kOob);
+  }
+  template <bool FINITE>
+  __device__ __forceinline__ void store(const Regs& r, char* S) const {
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = r.v[e / 4][e % 4];
+    uint4 q[3];
+    split_parts8<FINITE>(x, q);
+    if (slot < 0) return;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) reinterpret_cast<uint4*>(S)[slot + 2 * p] = q[p];
+  }
+};
+
+// As gemm_parts_tile, with both operands through registers and their loads two
+// steps ahead: B streams from HBM, and with one step in flight (8 KB a
+// workgroup) the latency of its loads would bound the kernel.
+template <int MT, int NT>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+    k_dense_parts(const typename DSplit<MT>::Params pa, const typename DSplit<NT>::Params pb,
+                  const EpiRowMajor::Params pe, TileGrid tg, uint32_t ktiles, uint32_t splits) {
+  using LA = DSplit<MT>;
+  using LB = DSplit<NT>;
+  using SA = typename LA::St;
+  using SB = typename LB::St;
+  constexpr int WM = MT / 2, WN = NT / 2, FM = WM / 32, FN = WN / 32;
+  constexpr int STAGE = SA::BYTES + SB::BYTES;
+  __shared__ __attribute__((aligned(16))) char S[2 * STAGE];
+  uint32_t mt, nt, z;
+  tile_coords(tg, mt, nt, z);
+  const uint32_t m0 = mt * MT, n0 = nt * NT;
+  const uint32_t kb = uint32_t((uint64_t(ktiles) * z) / splits);
+  const uint32_t ke = uint32_t((uint64_t(ktiles) * (z + 1)) / splits);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave / 2, wn = wave % 2;
+  LA la;
+  LB lb;
+  la.init(pa, m0, tid);
+  lb.init(pb, n0, tid);
+  f16v acc[FM][FN];
+
+  auto k_loop = [&](auto fp32) {
+    constexpr bool FP32 = decltype(fp32)::value;
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+    typename LA::Regs ra[2];
+    typename LB::Regs rb[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      la.load(kb + s, ke, ra[s]);
+      lb.load(kb + s, ke, rb[s]);
+    }
+    la.template store<!FP32>(ra[0], S);
+    lb.template store<!FP32>(rb[0], S + SA::BYTES);
+    __syncthreads();
+    // Step kt from stage `cur`, whose registers then take step kt + 2.
+    auto step = [&](uint32_t kt, auto curc) {
+      constexpr int cur = decltype(curc)::value;
+      const char* Ac = S + cur * STAGE;
+      la.load(kt + 2, ke, ra[cur]);
+      lb.load(kt + 2, ke, rb[cur]);
+      __builtin_amdgcn_sched_barrier(0);
+      u4v a[FM][3], b[FN][3];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) b[j][p] = SB::frag(Ac + SA::BYTES, p, wn * WN + 32 * j, lane);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) a[i][p] = SA::frag(Ac, p, wm * WM + 32 * i, lane);
+      }
+      parts_mma<FP32>(a, b, acc);
+      la.template store<!FP32>(ra[cur ^ 1], S + (cur ^ 1) * STAGE);
+      lb.template store<!FP32>(rb[cur ^ 1], S + (cur ^ 1) * STAGE + SA::BYTES);
+      __syncthreads();
+    };
+    for (uint32_t kt = kb; kt < ke; kt += 2) {
+      step(kt, std::integral_constant<int, 0>{});
+      if (kt + 1 < ke) step(kt + 1, std::integral_constant<int, 1>{});
+    }
+  };
+  k_loop(std::false_type{});
+  if (__syncthreads_or(parts_bad(acc))) k_loop(std::true_type{});
+  parts_store<PEpiRowMajor>(pe, acc, m0 + wm * WM, n0 + wn * WN, z, lane);
+}
+
+struct DensePartsRun {
+  const float *a, *b;
+  float *c, *part;
+  uint32_t M, K, N, ld, splits;
+  template <int MT, int NT>
+  int occ(bool) const {
+    return occupancy(k_dense_parts<MT, NT>);
+  }
+  template <int MT, int NT>
+  bool run() const {
+    const uint32_t kt = cdiv(K, 16);
+    const typename DSplit<MT>::Params pa{a, M, ld, M * ld};
+    const typename DSplit<NT>::Params pb{b, N, ld, N * ld};
+    const EpiRowMajor::Params pe{splits > 1 ? part : c, M, N, N, M * N};
+    const TileGrid tg{cdiv(M, MT), cdiv(N, NT), xcd_order() ? 1u : 0u};
+    hipLaunchKernelGGL((k_dense_parts<MT, NT>), dim3(tg.gm * tg.gn * splits), dim3(kThreads), 0,
+                       stream(), pa, pb, pe, tg, kt, splits);
+    return check_launch("gemm") && (splits == 1 || split_sum(part, c, M * N, splits));
+  }
+};
+#define DCE_DENSE_TILES DCE_T(128, 128) DCE_T(128, 64) DCE_T(64, 128) DCE_T(64, 64)
+template <class F>
+static bool dense_dispatch(const TileCfg& c, F&& f) {
+#define DCE_T(a, b) \
+  if (c.MT == a && c.NT == b) return f.template run<a, b>();
+  DCE_DENSE_TILES
+#undef DCE_T
+  set_error("gemm: unsupported tile %dx%d", c.MT, c.NT);
+  return false;
+}
+template <class F>
+static int dense_occ(const TileCfg& c, const F& f) {
+#define DCE_T(a, b) \
+  if (c.MT == a && c.NT == b) return f.template occ<a, b>(c.splits > 1);
+  DCE_DENSE_TILES
+#undef DCE_T
+  return 1;
+}
+
+// More than one 64-row tile and at least 2e9 products: 96 x 4096 x 4096 44 ->
+// 40, 200 x 4096 x 4096 86 -> 66, 320 x 9000 x 700 (rows x columns x K) 58 ->
+// 41, 512 x 1500 x 4096 66 -> 55 us; 256 x 2048 x 2048 (33 -> 34) and 200 x 700
+// x 900 (12.5 -> 14.4 us) stay on fp32 MFMAs.  Over many rows the dot products
+// have to be long as well: 500 x 4000 x 1200 loses (54 -> 59 us).
+static bool dense_on_parts(uint32_t M, uint32_t K, uint32_t N, bool aT, bool bT) {
+  return !aT && bT && M > 64 && K >= (M > 384 ? 2048u : 512u) && double(M) * N * K >= 2e9 &&
+         size_t(M) * N < kOob;
+}
+
 bool gemm(const float* a, const float* b, float* c, uint32_t M, uint32_t K, uint32_t N,
           uint32_t flags) {
   if (K == 0) return fill_zero(c, size_t(M) * N);
@@ -56,7 +238,10 @@ bool gemm(const float* a, const float* b, float* c, uint32_t M, uint32_t K, uint
     if (aT && !bT) return tiles_occ(t, GemmRun<true, false>{});
     return tiles_occ(t, GemmRun<true, true>{});
   };
-  TileCfg cfg = choose("DCE_TUNE_GEMM", M, N, pad4(K), 16, true, gemm_occ);
+  const bool parts = dense_on_parts(M, K, N, aT, bT);
+  TileCfg cfg = parts ? parts_choose("DCE_TUNE_GEMM", M, N, K, 16, true,
+                                     [&](const TileCfg& t) { return dense_occ(t, DensePartsRun{}); })
+                      : choose("DCE_TUNE_GEMM", M, N, pad4(K), 16, true, gemm_occ);
   // A grid that leaves CUs idle (small GEMMs such as AlexNet's fc3) runs
   // faster on 64 x 64 tiles 32 deep, at split counts that fill the chip:
   // fc3 forward 34 -> 22 us, its dA 29 -> 24 us in a sweep of every tile
@@ -65,7 +250,7 @@ bool gemm(const float* a, const float* b, float* c, uint32_t M, uint32_t K, uint
   auto wgs = [&](const TileCfg& t) {
     return cdiv(M, uint32_t(t.MT)) * cdiv(N, uint32_t(t.NT)) * t.splits;
   };
-  if (!getenv("DCE_TUNE_GEMM") && wgs(cfg) < cus && M >= 64 && N >= 64) {
+  if (!parts && !getenv("DCE_TUNE_GEMM") && wgs(cfg) < cus && M >= 64 && N >= 64) {
     const uint32_t kt32 = cdiv(pad4(K), 32u);
     TileCfg alt{64, 64, 32, 1};
     const uint32_t t64 = cdiv(M, 64u) * cdiv(N, 64u);
@@ -79,7 +264,7 @@ bool gemm(const float* a, const float* b, float* c, uint32_t M, uint32_t K, uint
   // 97 us, fc2 forward 56 -> 50 us, fc2 input gradient 53 -> 49 us in a sweep
   // of tiles and split counts on MI355X; wider grids, such as fc1's input
   // gradient with 288 such tiles, keep the model's choice).
-  if (!getenv("DCE_TUNE_GEMM") && M <= 128 && pad4(K) >= 4096) {
+  if (!parts && !getenv("DCE_TUNE_GEMM") && M <= 128 && pad4(K) >= 4096) {
     const uint32_t t64 = cdiv(M, 64u) * cdiv(N, 64u), kt32 = cdiv(pad4(K), 32u);
     if (t64 >= 64 && t64 <= 256) {
       TileCfg alt{64, 64, 32, std::max(1u, std::min(16u, 1024u / t64))};
@@ -111,7 +296,9 @@ bool gemm(const float* a, const float* b, float* c, uint32_t M, uint32_t K, uint
   {
     ProfScope prof("gemm", 2.0 * M * N * double(K),
                    4.0 * (double(M) * K + double(K) * N + double(M) * N));
-    if (!aT && !bT)
+    if (parts)
+      ok = dense_dispatch(cfg, DensePartsRun{ap, bp, c, part, M, K, N, lda, cfg.splits});
+    else if (!aT && !bT)
       ok = tiles_dispatch(cfg, GemmRun<false, false>{ap, bp, c, M, K, N, cfg.splits, lda, ldb, kdA, kdB, part});
     else if (!aT && bT)
       ok = tiles_dispatch(cfg, GemmRun<false, true>{ap, bp, c, M, K, N, cfg.splits, lda, ldb, kdA, kdB, part});

@@ -1,5 +1,6 @@
 // fp32 products on the bf16 matrix cores: the implicit GEMM of the
-// convolutions' backward passes (dce_igemm_dw.hip, dce_igemm_dx.hip).
+// convolutions' backward passes (dce_igemm_dw.hip, dce_igemm_dx.hip) and the
+// linear layers' input gradient (dce_igemm_dense.hip).
 //
 // A float has a 24-bit significand and three bf16 have 3 x 8: x = h + m + l
 // exactly, each part the upper half of what the ones before it leave (exact
@@ -349,6 +350,78 @@ struct PEpiPhase {
   }
 };
 
+// acc += a b for one 16-deep step: six bf16 products, or (FP32) the parts put
+// together again and multiplied in fp32.
+template <bool FP32, int FM, int FN>
+__device__ __forceinline__ void parts_mma(const u4v (&a)[FM][3], const u4v (&b)[FN][3],
+                                          f16v (&acc)[FM][FN]) {
+  if constexpr (!FP32) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      f16v t[FN];
+#pragma unroll
+      for (int j = 0; j < FN; ++j) t[j] = mfma_bf16(b[j][1], a[i][1], f16v{});
+#pragma unroll
+      for (int j = 0; j < FN; ++j) t[j] = mfma_bf16(b[j][0], a[i][2], t[j]);
+#pragma unroll
+      for (int j = 0; j < FN; ++j) t[j] = mfma_bf16(b[j][2], a[i][0], t[j]);
+#pragma unroll
+      for (int j = 0; j < FN; ++j) t[j] = mfma_bf16(b[j][0], a[i][1], t[j]);
+#pragma unroll
+      for (int j = 0; j < FN; ++j) t[j] = mfma_bf16(b[j][1], a[i][0], t[j]);
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] = mfma_bf16(b[j][0], a[i][0], acc[i][j]);
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] += t[j];
+    }
+  } else {
+    // Lane halves hold k = e and 8 + e: two k per fp32 MFMA.
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      auto word = [&](const u4v (&f)[3]) {
+        float x[3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+          x[p] = __uint_as_float(e & 1 ? f[p][e / 2] & 0xffff0000u : f[p][e / 2] << 16);
+        return (x[0] + x[1]) + x[2];
+      };
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(word(b[j]), word(a[i]), acc[i][j], 0, 0, 0);
+    }
+  }
+}
+// Does the tile hold an infinity or a NaN?
+template <int FM, int FN>
+__device__ __forceinline__ bool parts_bad(const f16v (&acc)[FM][FN]) {
+  // x * 0 is NaN for an infinity or a NaN.
+  float bad = 0.f;
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) bad = fmaf(acc[i][j][v], 0.f, bad);
+  return bad != bad;
+}
+template <class EPI, int FM, int FN>
+__device__ __forceinline__ void parts_store(const typename EPI::Params& pe, const f16v (&acc)[FM][FN],
+                                            uint32_t m0, uint32_t n0, uint32_t z, int lane) {
+  // Block (i, j): row m = lane % 32, columns 8q + 4 * (lane / 32) + 0 .. 3.
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        EPI::quad(pe, m0 + 32 * i + (lane & 31),
+                  n0 + 32 * j + 8 * q + 4 * (lane >> 5), z,
+                  f4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
+                     acc[i][j][4 * q + 3]});
+}
+
 // ---------------------------------------------------------------------------
 // The kernel: 256 threads, waves 2 x 2 (1 x 4 when the tile is four times as
 // wide as high, or 32 rows high) over an MT x NT tile of 32 x 32 blocks; K in
@@ -411,69 +484,15 @@ __device__ __forceinline__ void gemm_parts_tile(char* S, const typename LA::Para
         la.issue(la, kt + 1, S + (cur ^ 1) * STAGE);
         lb.issue(lb, kt + 1, S + (cur ^ 1) * STAGE + SA::BYTES);
       }
-      if constexpr (!FP32) {
-#pragma unroll
-        for (int i = 0; i < FM; ++i) {
-          f16v t[FN];
-#pragma unroll
-          for (int j = 0; j < FN; ++j) t[j] = mfma_bf16(b[j][1], a[i][1], f16v{});
-#pragma unroll
-          for (int j = 0; j < FN; ++j) t[j] = mfma_bf16(b[j][0], a[i][2], t[j]);
-#pragma unroll
-          for (int j = 0; j < FN; ++j) t[j] = mfma_bf16(b[j][2], a[i][0], t[j]);
-#pragma unroll
-          for (int j = 0; j < FN; ++j) t[j] = mfma_bf16(b[j][0], a[i][1], t[j]);
-#pragma unroll
-          for (int j = 0; j < FN; ++j) t[j] = mfma_bf16(b[j][1], a[i][0], t[j]);
-#pragma unroll
-          for (int j = 0; j < FN; ++j) acc[i][j] = mfma_bf16(b[j][0], a[i][0], acc[i][j]);
-#pragma unroll
-          for (int j = 0; j < FN; ++j) acc[i][j] += t[j];
-        }
-      } else {
-        // Lane halves hold k = e and 8 + e: two k per fp32 MFMA.
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          auto word = [&](const u4v (&f)[3]) {
-            float x[3];
-#pragma unroll
-            for (int p = 0; p < 3; ++p)
-              x[p] = __uint_as_float(e & 1 ? f[p][e / 2] & 0xffff0000u : f[p][e / 2] << 16);
-            return (x[0] + x[1]) + x[2];
-          };
-#pragma unroll
-          for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(word(b[j]), word(a[i]), acc[i][j], 0, 0, 0);
-        }
-      }
+      parts_mma<FP32>(a, b, acc);
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
     }
   };
   k_loop(std::false_type{});
-  // x * 0 is NaN for an infinity or a NaN.
-  float bad = 0.f;
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) bad = fmaf(acc[i][j][v], 0.f, bad);
-  if (__syncthreads_or(bad != bad)) k_loop(std::true_type{});
-  // Block (i, j): row m = lane % 32, columns 8q + 4 * (lane / 32) + 0 .. 3.
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        EPI::quad(pe, m0 + wm * WM + 32 * i + (lane & 31),
-                  n0 + wn * WN + 32 * j + 8 * q + 4 * (lane >> 5), z,
-                  f4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
-                     acc[i][j][4 * q + 3]});
+  if (__syncthreads_or(parts_bad(acc))) k_loop(std::true_type{});
+  parts_store<EPI>(pe, acc, m0 + wm * WM, n0 + wn * WN, z, lane);
 }
 
 template <int MT, int NT, class LA, class LB, class EPI>

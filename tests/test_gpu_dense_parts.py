@@ -1,0 +1,65 @@
+"""Large A B^T products of MatMulAlloc (a linear layer's input gradient) on bf16
+parts, at tile edges and ragged sizes, and with operands that are not finite,
+against the float64 oracle.
+
+Bound per element, as for the convolutions on parts: with S the same sum over
+magnitudes, the dropped part products are below 3 * 2^-21 S, and each step of 16
+rounds at most eight times by 2^-24 of a partial sum; split-K adds one rounding
+per split (at most 16)."""
+import numpy as np
+import pytest
+
+from oracle import kernels as K
+from tests.helpers import download, release, rng, upload
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    # M, K, N: at least 2e9 products, M > 64, K >= 512 (2048 past 384 rows)
+    (65, 5200, 6001),      # one row past a tile, one column past one
+    (128, 4096, 3840),     # whole tiles
+    (129, 4099, 3901),     # K pads its rows to 4 and its last step to 16
+    (384, 512, 10200),     # the shortest dot products
+    (385, 2048, 2600),     # and beyond 384 rows
+    (200, 100001, 101),    # few columns, long K
+]
+
+
+def _matmul(eng, a, b):
+    (M, Kd), N = a.shape, b.shape[0]
+    ha, hb = upload(eng, a), upload(eng, b)
+    hc = eng.lib.MatMulAlloc(ha, hb, M, Kd, N, 2)
+    assert hc, eng.last_error()
+    c = download(eng, hc, (M, N))
+    release(eng, ha, hb, hc)
+    return c
+
+
+@pytest.mark.parametrize("M,Kd,N", SHAPES)
+def test_a_bt_on_parts(eng, M, Kd, N):
+    r = rng(M + Kd + N)
+    a = r.standard_normal((M, Kd), dtype=np.float32)
+    b = r.standard_normal((N, Kd), dtype=np.float32)
+    ref = K.matmul(a, b, M, Kd, N, 2)
+    S = K.matmul(np.abs(a), np.abs(b), M, Kd, N, 2)
+    bound = (3 * 2.0 ** -21 + (8 * (Kd / 16 + 2) + 16) * 2.0 ** -24) * S
+    assert np.all(np.abs(_matmul(eng, a, b) - ref) <= bound)
+
+
+def test_a_bt_not_finite(eng):
+    M, Kd, N = 130, 4100, 3800
+    r = rng(5)
+    a = r.standard_normal((M, Kd), dtype=np.float32)
+    b = r.standard_normal((N, Kd), dtype=np.float32)
+    a[3, 17], a[129, 4099], b[700, 5], b[3799, 2000] = np.inf, np.nan, -np.inf, np.nan
+    b[64, 9] = np.array([0x7F800001], np.uint32).view(np.float32)[0]  # payload in the low half alone
+    a[70, 40], b[:, 40], b[700, 40] = 3e38, 1e5, 1.0  # row 70 overflows but beside the infinity
+    with np.errstate(all="ignore"):
+        ref = K.matmul(a, b, M, Kd, N, 2).astype(np.float32)
+    c = _matmul(eng, a, b)
+    assert np.array_equal(np.isnan(c), np.isnan(ref))
+    inf = np.isinf(ref)
+    assert np.array_equal(np.isinf(c), inf)
+    assert np.array_equal(c[inf], ref[inf])
+    fin = np.isfinite(ref)
+    assert np.max(np.abs(c[fin] - ref[fin])) <= 1e-5 * np.max(np.abs(ref[fin]))
