@@ -258,6 +258,18 @@ bool gemm(const float* a, const float* b, float* c, uint32_t M, uint32_t K, uint
     while (t64 * alt.splits < cus && alt.splits < 16 && kt32 / (alt.splits + 1) >= 8) alt.splits++;
     if (wgs(alt) > wgs(cfg)) cfg = alt;
   }
+  // A^T B over few rows (a linear layer's filter gradient): a 128 x 128 tile is
+  // 16 steps at most, and a last batch of four workgroups a CU that is not full
+  // costs as much as a full one.  64 x 128 tiles halve what is lost: 9216 x
+  // 128 x 4096 (rows x K x columns; 2.25 batches) 106 -> 99 us, 5120 x 128 x
+  // 4096 70 -> 57, 9216 x 250 x 1000 54 -> 46, 4608 x 37 x 4096 32 -> 25 us.
+  // Grids that fill their batches stay (4096 x 128 x 4096 42 -> 44, 8192 x 250
+  // x 4096 137 -> 139 us).  The order of every sum is the same.
+  if (!getenv("DCE_TUNE_GEMM") && aT && !bT && K <= 256 && cfg.splits == 1 && cfg.MT == 128 &&
+      cfg.NT == 128) {
+    const uint32_t t = wgs(cfg), batch = cus * uint32_t(gemm_occ(cfg));
+    if (double(cdiv(t, batch)) * batch > 1.1 * t) cfg.MT = 64;
+  }
   // Skinny products with long dot products (a linear layer's forward and
   // input gradient at batch 128): 64 x 64 tiles 32 deep over about 1024
   // workgroups beat the 128 x 128 split-K choice (AlexNet fc1 forward 104 ->
