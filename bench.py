@@ -913,10 +913,11 @@ def main():
             "bound": "mfma",
             "kernel": "conv backward of all layers, each ConvBackwardFused call whole: G pass "
                       "k_to_nhwc (ReLU mask + NHWC transpose + bias partials, with the dX filter "
-                      "re-layout as extra blocks; k_mask_pad for c1), dW k_igemm<LdGradKR,LdXTapKR> "
+                      "re-layout as extra blocks; k_mask_pad for c1), dW k_gemm_parts<PGrad,PTap> "
                       "(c1, C = 3: k_igemm<LdGPadRK,LdPsRK> on the stride-phase copy) + k_dw_final "
-                      "(with the bias-gradient sum as extra blocks), dX k_igemm<LdDenseRK,LdPixRK> "
-                      "(+ k_splitk_nchw4 when split)",
+                      "(with the bias-gradient sum as extra blocks), dX k_gemm_parts<PRows,PPix> "
+                      "(+ k_splitk_nchw4 when split); k_gemm_parts takes six bf16 MFMA products per "
+                      "fp32 product, so the fp32 MFMA peak quoted is passed",
             "achieved": round(achieved, 3),
             "peak": MFMA_FP32_PEAK_TFLOPS,
             "unit": "TFLOP/s",
