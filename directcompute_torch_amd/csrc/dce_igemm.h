@@ -1333,11 +1333,13 @@ constexpr int igemm_min_waves() {
   return MT * NT == 128 * 128 ? 4 : (MT * NT == 256 * 128 ? 2 : 1);
 }
 
+// One MT x NT tile at (m0, n0) over the K tiles [kb, ke); As and Bs are two LDS
+// stages of each operand.
 template <int MT, int NT, int KT, class LA, class LB, class EPI>
-__global__ void __launch_bounds__(kThreads)
-    __attribute__((amdgpu_waves_per_eu(igemm_min_waves<MT, NT>())))
-    k_igemm(const typename LA::Params pa, const typename LB::Params pb,
-            const typename EPI::Params pe, TileGrid tg, uint32_t ktiles, uint32_t splits) {
+__device__ __forceinline__ void igemm_tile(float* As, float* Bs, const typename LA::Params& pa,
+                                           const typename LB::Params& pb,
+                                           const typename EPI::Params& pe, uint32_t m0, uint32_t n0,
+                                           uint32_t z, uint32_t kb, uint32_t ke) {
   using SA = typename LA::St;
   using SB = typename LB::St;
   // WKS (narrow tiles, MT <= 32 with KT = 64): the four waves split every K
@@ -1348,18 +1350,11 @@ __global__ void __launch_bounds__(kThreads)
   constexpr int WGM = WKS ? 1 : (MT >= 64 ? 2 : 1), WGN = WKS ? 1 : 4 / WGM;  // wave grid
   constexpr int WM = MT / WGM, WN = NT / WGN, FM = WM / 16, FN = WN / 16;
   static_assert(FM >= 1 && FN >= 1 && WM % 16 == 0 && WN % 16 == 0, "tile too small");
-  __shared__ __attribute__((aligned(16))) float As[2 * SA::SIZE];
-  __shared__ __attribute__((aligned(16))) float Bs[2 * SB::SIZE];
   static_assert(!WKS || 3 * FM * FN * 256 <= 2 * SB::SIZE, "wave partials fit the B stages");
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int wm = WKS ? 0 : wave / WGN, wn = WKS ? 0 : wave % WGN;  // WKS: every wave the whole tile
-  uint32_t mt, nt, z;
-  tile_coords(tg, mt, nt, z);
-  const uint32_t m0 = mt * MT, n0 = nt * NT;
-  const uint32_t kb = uint32_t((uint64_t(ktiles) * z) / splits);
-  const uint32_t ke = uint32_t((uint64_t(ktiles) * (z + 1)) / splits);
 
   LA la;
   LB lb;
@@ -1475,11 +1470,58 @@ __global__ void __launch_bounds__(kThreads)
         for (int j = 0; j < FN; ++j) acc[i][j] += red[(w * FM * FN + i * FN + j) * 64 + lane];
   }
   if constexpr (EpiStats<EPI>::value) {
-    static_assert(WGN * 4 * MT * 8 <= int(sizeof(As)), "the statistics' lane sums fit the A stages");
+    static_assert(WGN * 4 * MT * 8 <= 2 * SA::SIZE * 4, "the statistics' lane sums fit the A stages");
     EPI::template store_stats<MT, NT, FM, FN, TACC, RA, RB, WGN>(pe, acc, m0, n0, wm, wn, lane, As);
   } else {
     EPI::template store<MT, NT, FM, FN, TACC, RA, RB>(pe, acc, m0, n0, z, wm, wn, lane);
   }
+}
+
+template <int MT, int NT, int KT, class LA, class LB, class EPI>
+__global__ void __launch_bounds__(kThreads)
+    __attribute__((amdgpu_waves_per_eu(igemm_min_waves<MT, NT>())))
+    k_igemm(const typename LA::Params pa, const typename LB::Params pb,
+            const typename EPI::Params pe, TileGrid tg, uint32_t ktiles, uint32_t splits) {
+  __shared__ __attribute__((aligned(16))) float As[2 * LA::St::SIZE];
+  __shared__ __attribute__((aligned(16))) float Bs[2 * LB::St::SIZE];
+  uint32_t mt, nt, z;
+  tile_coords(tg, mt, nt, z);
+  igemm_tile<MT, NT, KT, LA, LB, EPI>(As, Bs, pa, pb, pe, mt * MT, nt * NT, z,
+                                      uint32_t((uint64_t(ktiles) * z) / splits),
+                                      uint32_t((uint64_t(ktiles) * (z + 1)) / splits));
+}
+
+// Up to four independent products of one shape of tile in one launch (the
+// sub-pixel phases of a stride-2 dX, each a quarter of the chip's work).
+constexpr int kMulti = 4;
+template <class LA, class LB, class EPI>
+struct Multi {
+  typename LA::Params pa[kMulti];
+  typename LB::Params pb[kMulti];
+  typename EPI::Params pe[kMulti];
+  uint32_t ktiles[kMulti], gm, first[kMulti + 1];  // first workgroup of each product
+};
+template <int MT, int NT, int KT, class LA, class LB, class EPI>
+__global__ void __launch_bounds__(kThreads)
+    __attribute__((amdgpu_waves_per_eu(igemm_min_waves<MT, NT>())))
+    k_igemm_multi(const Multi<LA, LB, EPI> a) {
+  __shared__ __attribute__((aligned(16))) float As[2 * LA::St::SIZE];
+  __shared__ __attribute__((aligned(16))) float Bs[2 * LB::St::SIZE];
+  const uint32_t id = xcd_block_id();
+  typename LA::Params pa = a.pa[0];
+  typename LB::Params pb = a.pb[0];
+  typename EPI::Params pe = a.pe[0];
+  uint32_t kt = a.ktiles[0], t = id;
+#pragma unroll
+  for (int i = 1; i < kMulti; ++i)
+    if (id >= a.first[i]) {
+      pa = a.pa[i];
+      pb = a.pb[i];
+      pe = a.pe[i];
+      kt = a.ktiles[i];
+      t = id - a.first[i];
+    }
+  igemm_tile<MT, NT, KT, LA, LB, EPI>(As, Bs, pa, pb, pe, t % a.gm * MT, t / a.gm * NT, 0, 0, kt);
 }
 
 // Filters in the K order of the pixel loaders (flat or blocked), zero for

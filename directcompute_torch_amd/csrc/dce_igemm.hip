@@ -1477,15 +1477,24 @@ bool conv_backward(const float* dy, const float* y, const float* x, const float*
   // A dX at stride 3 or more runs as sub-pixel phases (conv_dx_phased), each with
   // its own filter re-layout and no split: the strided gather would walk
   // s^2 times the taps that reach a pixel (AlexNet c1's dX at b128: 18.0 ->
-  // 1.24 ms).  At stride 2 the gather's 4x is about what the phases' extra
-  // launches and smaller, unsplit grids cost (ResNet-like layers of 0.4-7
-  // GFLOP measured from 40 % faster to 65 % slower), so it stays.
-  // On parts the four stride-2 phases share one launch and are taken too (12 x
-  // 37 x 61 x 45 -> 70, k5: dX 78 -> 32 us).
-  const bool phased = dx && (g.s >= 3 || (parts && g.s == 2));
+  // 1.24 ms).  At stride 2 the four phases share one launch.  On parts they are
+  // always taken (12 x 37 x 61 x 45 -> 70, k5: dX 78 -> 32 us).  On fp32 MFMAs
+  // (forward and backward, gather -> phases; B x C x H x W -> OC): 128 x 8 x
+  // 100 x 90 -> 40, k3 338 -> 229, 32 x 16 x 112 x 112 -> 24, k3 102 -> 85, 20
+  // x 160 x 160 -> 31, k5 75 -> 58, 64 x 128 x 28 x 28 -> 256, k1 104 -> 84 us.
+  // Not where the gather splits its k * k taps so often that the largest
+  // phase's unsplit taps, (k + 1) / 2 squared, make the longer chain (30 x 9 x
+  // 9 -> 384, k5 79 -> 131, 128 x 30 x 7 x 7 -> 384, k5 149 -> 180 us), nor
+  // where the products saved do not pay for the launches added, the filters'
+  // and for k = 1 the zeros' (8 x 16 x 64 x 64 -> 24, k3 37 -> 41, 16 x 64 x
+  // 56 x 56 -> 128, k1 alone 76 -> 88 us).
+  bool phased = dx && (g.s >= 3 || (parts && g.s == 2));
   if (dx && !phased) {
     dxc = conv_dx_choose(g, parts);
-    nQ = dxc.splits > 1 ? size_t(dxc.splits) * g.C * g.B * HW : 0;
+    const uint32_t kp = (g.k + 1) / 2;
+    const double products = double(g.C) * g.B * HW * KK * OCp;
+    phased = g.s == 2 && dxc.splits * kp * kp <= KK && products >= (g.k == 1 ? 8e8 : 2e8);
+    if (!phased) nQ = dxc.splits > 1 ? size_t(dxc.splits) * g.C * g.B * HW : 0;
   }
   if (dx) nW = al64(wFloats);
   float* ws = workspace(nG + nGp + nDb + nX + nP + nW + nQ);

@@ -51,6 +51,18 @@ struct PhaseGeom {
   uint32_t ph, pw, rh, rw, nh, nw, qh, qw, GH, GW;
 };
 
+template <class LA, class LB, bool BLK>
+static void dx_phase_params(const float* wt, const float* gn, float* dx, const ConvGeom& g,
+                            const PhaseGeom& q, typename LA::Params& pa, typename LB::Params& pb,
+                            EpiNCHWPhase::Params& pe) {
+  const uint32_t OCp = pad4(g.OC), KK = q.nh * q.nw, kdim = KK * OCp;
+  const uint32_t GHW = q.GH * q.GW, N = g.B * GHW;
+  pa = {wt, kdim, g.C, kdim, g.C * kdim};
+  pb = {gn, g.OH, g.OW, OCp, q.nw, 1, q.qh, q.GW, GHW, N, kdim,
+        g.B * g.OH * g.OW * OCp, make_fastdiv(GHW), make_fastdiv(q.GW),
+        make_fastdiv(BLK ? KK : OCp), make_fastdiv(q.nw), int(q.qw) - int(q.qh)};
+  pe = {dx, g.C, g.H, g.W, q.GW, GHW, N, g.s, q.ph, q.pw, make_fastdiv(GHW), make_fastdiv(q.GW)};
+}
 template <bool BLK>
 struct DxPhaseRun {
   const float* wt;
@@ -65,17 +77,13 @@ struct DxPhaseRun {
   }
   template <int MT, int NT, int KT>
   bool run() {
-    const uint32_t OCp = pad4(g.OC), KK = q.nh * q.nw, kdim = KK * OCp;
-    const uint32_t GHW = q.GH * q.GW, N = g.B * GHW;
     using LA = LdDenseRK<MT, KT>;
     using LB = LdPixRK<NT, KT, false, true, BLK>;
-    const typename LA::Params pa{wt, kdim, g.C, kdim, g.C * kdim};
-    const typename LB::Params pb{gn, g.OH, g.OW, OCp, q.nw, 1, q.qh, q.GW, GHW, N, kdim,
-                                 g.B * g.OH * g.OW * OCp, make_fastdiv(GHW), make_fastdiv(q.GW),
-                                 make_fastdiv(BLK ? KK : OCp), make_fastdiv(q.nw),
-                                 int(q.qw) - int(q.qh)};
-    const EpiNCHWPhase::Params pe{dx, g.C, g.H, g.W, q.GW, GHW, N, g.s, q.ph, q.pw,
-                                  make_fastdiv(GHW), make_fastdiv(q.GW)};
+    typename LA::Params pa;
+    typename LB::Params pb;
+    EpiNCHWPhase::Params pe;
+    dx_phase_params<LA, LB, BLK>(wt, gn, dx, g, q, pa, pb, pe);
+    const uint32_t kdim = q.nh * q.nw * pad4(g.OC), N = g.B * q.GH * q.GW;
     return launch<MT, NT, KT, LA, LB, EpiNCHWPhase>(pa, pb, pe, g.C, N, cdiv(kdim, KT), 1,
                                                     "conv_backward_input");
   }
@@ -126,49 +134,82 @@ struct DxPartsRun {
   }
 };
 
-// The four phases of a stride-2 dX on parts in one launch, their filters
-// re-laid by another; phases that no tap reaches (k = 1) are zero.
-struct DxMulti {
-  using EPI = PEpiPhase;
+// The phases of a stride-2 dX that some tap reaches, in one launch.
+struct DxPhases {
   const float* gn;
   float* dx;
   ConvGeom g;
   PhaseGeom q[4];
   const float* wt[4];
   uint32_t n;
+  // f(i, phase, columns) fills product i; returns the workgroups of them all.
+  template <class A, class F>
+  uint32_t fill(A& a, uint32_t MT, uint32_t NT, F&& f) const {
+    a.gm = cdiv(g.C, MT);
+    uint32_t wgs = 0;
+    for (uint32_t i = 0; i < 4; ++i) {
+      a.first[i] = i < n ? wgs : 0xFFFFFFFFu;
+      if (i >= n) continue;
+      const uint32_t N = g.B * q[i].GH * q[i].GW;
+      f(i, q[i], N);
+      wgs += a.gm * cdiv(N, NT);
+    }
+    return wgs;
+  }
+};
+struct DxMultiParts : DxPhases {
+  using EPI = PEpiPhase;
   template <int MT, int NT>
   int occ(bool) const {
     return occupancy(k_gemm_parts_multi<MT, NT, PRows<MT>, PPix<NT, true>, EPI>);
   }
   template <int MT, int NT>
   bool run() const {
-    PMulti<PRows<MT>, PPix<NT, true>, EPI> a{};
+    Multi<PRows<MT>, PPix<NT, true>, EPI> a{};
     const uint32_t no = pad16(g.OC) / 16;
-    a.gm = cdiv(g.C, MT);
-    uint32_t wgs = 0;
-    for (uint32_t i = 0; i < 4; ++i) {
-      a.first[i] = i < n ? wgs : 0xFFFFFFFFu;
-      if (i >= n) continue;
-      const PhaseGeom& f = q[i];
-      const uint32_t KK = f.nh * f.nw, GHW = f.GH * f.GW, N = g.B * GHW;
+    const uint32_t wgs = fill(a, MT, NT, [&](uint32_t i, const PhaseGeom& f, uint32_t N) {
+      const uint32_t KK = f.nh * f.nw, GHW = f.GH * f.GW;
       a.ktiles[i] = KK * no;
       a.pa[i] = {wt[i], g.C, KK * no, g.C * KK * no * 24};
       a.pb[i] = {gn, g.OH, g.OW, no, f.nw, 1, f.qh, f.GW, GHW, N,
                  uint32_t(parts_floats(size_t(g.B) * g.OH * g.OW, g.OC)), make_fastdiv(GHW),
                  make_fastdiv(f.GW), make_fastdiv(KK), make_fastdiv(f.nw), int(f.qw) - int(f.qh)};
       a.pe[i] = {dx, g.C, g.H, g.W, f.GW, GHW, N, g.s, f.ph, f.pw, a.pb[i].dGridHW, a.pb[i].dGridW};
-      wgs += a.gm * cdiv(N, NT);
-    }
+    });
     hipLaunchKernelGGL((k_gemm_parts_multi<MT, NT, PRows<MT>, PPix<NT, true>, EPI>), dim3(wgs),
                        dim3(kThreads), 0, stream(), a);
     return check_launch("conv_backward_input");
   }
 };
+template <bool BLK>
+struct DxMulti : DxPhases {
+  template <int MT, int NT, int KT>
+  int occ(bool) const {
+    return occupancy(k_igemm_multi<MT, NT, KT, LdDenseRK<MT, KT>, LdPixRK<NT, KT, false, true, BLK>,
+                                   EpiNCHWPhase>);
+  }
+  template <int MT, int NT, int KT>
+  bool run() const {
+    using LA = LdDenseRK<MT, KT>;
+    using LB = LdPixRK<NT, KT, false, true, BLK>;
+    Multi<LA, LB, EpiNCHWPhase> a{};
+    const uint32_t wgs = fill(a, MT, NT, [&](uint32_t i, const PhaseGeom& f, uint32_t N) {
+      a.ktiles[i] = cdiv(f.nh * f.nw * pad4(g.OC), KT);
+      dx_phase_params<LA, LB, BLK>(wt[i], gn, dx, g, f, a.pa[i], a.pb[i], a.pe[i]);
+    });
+    hipLaunchKernelGGL((k_igemm_multi<MT, NT, KT, LA, LB, EpiNCHWPhase>), dim3(wgs), dim3(kThreads),
+                       0, stream(), a);
+    return check_launch("conv_backward_input");
+  }
+};
+// Their filters are re-laid by one launch too; phases that no tap reaches (k =
+// 1) are zero.
 template <class Geom>
 static bool phases_in_one(const float* w, float* wt, const float* gn, float* dx, const ConvGeom& g,
-                          Geom&& geom) {
-  const uint32_t OCp = pad16(g.OC);
-  DxMulti m{};
+                          bool parts, Geom&& geom) {
+  const uint32_t OCp = parts ? pad16(g.OC) : pad4(g.OC);
+  const bool blk = blocked_k(OCp);
+  DxPhases m{};
   m.gn = gn;
   m.dx = dx;
   m.g = g;
@@ -184,19 +225,31 @@ static bool phases_in_one(const float* w, float* wt, const float* gn, float* dx,
       empty = true;
       continue;
     }
-    pw.p[m.n] = WPerm{w, at, g.OC, g.C, KK, OCp, KK * OCp, 1, 1, q.nw, g.k, 2, q.rh, q.rw, 1u};
+    pw.p[m.n] = WPerm{w, at, g.OC, g.C, KK, OCp, KK * OCp, 1, blk ? 1 : 0, q.nw, g.k, 2, q.rh, q.rw,
+                      parts ? 1u : 0u};
     m.wt[m.n] = at;
     m.q[m.n++] = q;
-    at += parts_floats(size_t(g.C) * KK, g.OC);
+    at += parts ? parts_floats(size_t(g.C) * KK, g.OC) : size_t(g.C) * KK * OCp;
     cols += g.B * q.GH * q.GW;
     kmax = std::max(kmax, KK * OCp);
   }
   if (empty && !fill_zero(dx, size_t(g.B) * g.C * g.H * g.W)) return false;
   if (m.n == 0) return true;
   if (!permute_w4(pw)) return false;
-  const TileCfg t = parts_choose("DCE_TUNE_DX", g.C, cols, kmax, 1, true,
-                                 [&](const TileCfg& v) { return parts_occ(v, m); });
-  return parts_dispatch(t, m);
+  if (parts) {
+    const DxMultiParts r{m};
+    const TileCfg t = parts_choose("DCE_TUNE_DX", g.C, cols, kmax, 1, true,
+                                   [&](const TileCfg& v) { return parts_occ(v, r); });
+    return parts_dispatch(t, r);
+  }
+  auto go = [&](const auto& r) {
+    TileCfg c = choose("DCE_TUNE_DX", g.C, cols, kmax, 1, true,
+                       [&](const TileCfg& t) { return tiles_occ16(t, r); }, true);
+    narrow_short_k(c, "DCE_TUNE_DX", g.C, cols, kmax);
+    c.splits = 1;
+    return tiles_dispatch16(c, r);
+  };
+  return blk ? go(DxMulti<true>{m}) : go(DxMulti<false>{m});
 }
 
 // dX of a strided convolution as its s*s sub-pixel phases: every input pixel
@@ -222,7 +275,7 @@ bool conv_dx_phased(const float* w, float* wt, const float* gn, float* dx, const
     q.qw = (pw + g.p - q.rw) / s;
     return q;
   };
-  if (parts && s == 2) return phases_in_one(w, wt, gn, dx, g, geom);
+  if (s == 2) return phases_in_one(w, wt, gn, dx, g, parts, geom);
   bool empty = false;
   for (uint32_t ph = 0; ph < s; ++ph)
     for (uint32_t pw = 0; pw < s; ++pw) {

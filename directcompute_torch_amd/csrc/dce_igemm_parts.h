@@ -507,19 +507,10 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
                                        uint32_t((uint64_t(ktiles) * (z + 1)) / splits));
 }
 
-// Up to four independent products of one shape of tile in one launch (the
-// sub-pixel phases of a stride-2 dX, each a quarter of the chip's work).
-constexpr int kPartsMulti = 4;
-template <class LA, class LB, class EPI>
-struct PMulti {
-  typename LA::Params pa[kPartsMulti];
-  typename LB::Params pb[kPartsMulti];
-  typename EPI::Params pe[kPartsMulti];
-  uint32_t ktiles[kPartsMulti], gm, first[kPartsMulti + 1];  // first workgroup of each product
-};
+// Up to four products in one launch, as k_igemm_multi.
 template <int MT, int NT, class LA, class LB, class EPI>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
-    k_gemm_parts_multi(const PMulti<LA, LB, EPI> a) {
+    k_gemm_parts_multi(const Multi<LA, LB, EPI> a) {
   __shared__ __attribute__((aligned(16))) char S[2 * PTile<MT, NT, LA, LB>::BYTES];
   const uint32_t id = xcd_block_id();
   typename LA::Params pa = a.pa[0];
@@ -527,7 +518,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
   typename EPI::Params pe = a.pe[0];
   uint32_t kt = a.ktiles[0], t = id;
 #pragma unroll
-  for (int i = 1; i < kPartsMulti; ++i)
+  for (int i = 1; i < kMulti; ++i)
     if (id >= a.first[i]) {
       pa = a.pa[i];
       pb = a.pb[i];
