@@ -1803,52 +1803,64 @@ static inline size_t al64(size_t n) { return (n + 63) & ~size_t(63); }
 inline uint32_t pad16(uint32_t c) { return (c + 15u) & ~15u; }
 // Floats of a [rows][pad16(c)] array of bf16 parts (96 bytes per 16 values).
 inline size_t parts_floats(size_t rows, uint32_t c) { return rows * (pad16(c) / 16) * 24; }
-// x as bf16 parts (dce_igemm_parts.h), each in the upper half of a word.  An
-// infinity or a NaN (made quiet, so that its upper half is one) has no m, l.
-struct Parts {
+// The bf16 parts (dce_igemm_parts.h) of two values, the first in the low half of
+// each word.  Every part is what the ones before it leave, rounded to nearest
+// even.  A value that rounds to infinity, an infinity or a NaN gets a NaN or
+// infinite part.
+using bf2 = __bf16 __attribute__((ext_vector_type(2)));
+struct Parts2 {
   uint32_t h, m, l;
 };
-__device__ __forceinline__ Parts split_parts(float x) {
-  uint32_t u = __float_as_uint(x);
-  if (x != x) u |= 0x00400000u;
-  const uint32_t hu = u & 0xffff0000u;
-  const bool fin = (u & 0x7f800000u) != 0x7f800000u;
-  const float r = x - __uint_as_float(hu);
-  const uint32_t mu = fin ? __float_as_uint(r) : 0u;
-  const float s = r - __uint_as_float(mu & 0xffff0000u);
-  return Parts{u, mu, fin ? __float_as_uint(s) : 0u};
+__device__ __forceinline__ uint32_t bf16_pair(float x, float y) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{x, y}, bf2));
 }
-
-// For finite x alone (4 instead of 12 instructions); others get a NaN as m.
-__device__ __forceinline__ Parts split_finite(float x) {
-  const uint32_t u = __float_as_uint(x);
-  const float r = x - __uint_as_float(u & 0xffff0000u);
-  const uint32_t mu = __float_as_uint(r);
-  return Parts{u, mu, __float_as_uint(r - __uint_as_float(mu & 0xffff0000u))};
+__device__ __forceinline__ Parts2 split_pair(float x, float y) {
+  const uint32_t h = bf16_pair(x, y);
+  const float rx = x - __uint_as_float(h << 16), ry = y - __uint_as_float(h & 0xffff0000u);
+  const uint32_t m = bf16_pair(rx, ry);
+  return Parts2{h, m, bf16_pair(rx - __uint_as_float(m << 16), ry - __uint_as_float(m & 0xffff0000u))};
 }
-// Parts of 8 values as one 16-byte quad per part.
+// x has no three finite bf16 parts: it is kept as a NaN, then its own upper and
+// lower half (parts_value puts it together again).
+__device__ __forceinline__ bool parts_raw(float x) {
+  return (__float_as_uint(x) & 0x7fffffffu) >= 0x7f7f8000u;
+}
+// Parts of 8 values as one 16-byte quad per part.  FINITE: nothing is raw (if
+// something is, it gets a NaN part).
 template <bool FINITE>
 __device__ __forceinline__ void split_parts8(const float (&x)[8], uint4 (&out)[3]) {
-  uint32_t h[8], m[8], l[8];
+  uint32_t q[3][4];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const Parts q = FINITE ? split_finite(x[e]) : split_parts(x[e]);
-    h[e] = q.h;
-    m[e] = q.m;
-    l[e] = q.l;
+  for (int e = 0; e < 4; ++e) {
+    const Parts2 p = split_pair(x[2 * e], x[2 * e + 1]);
+    q[0][e] = p.h;
+    q[1][e] = p.m;
+    q[2][e] = p.l;
   }
-  auto pack = [](const uint32_t (&u)[8]) {
-    uint4 v;
-    v.x = __builtin_amdgcn_perm(u[1], u[0], 0x07060302u);
-    v.y = __builtin_amdgcn_perm(u[3], u[2], 0x07060302u);
-    v.z = __builtin_amdgcn_perm(u[5], u[4], 0x07060302u);
-    v.w = __builtin_amdgcn_perm(u[7], u[6], 0x07060302u);
-    return v;
-  };
-  out[0] = pack(h);
-  out[1] = pack(m);
-  out[2] = pack(l);
+  if constexpr (!FINITE) {
+    bool raw = false;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) raw |= parts_raw(x[e]);
+    if (raw) {  // hardly ever
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (!parts_raw(x[e])) continue;
+        const uint32_t u = __float_as_uint(x[e]), at = 16 * (e & 1), keep = 0xffff0000u >> at;
+        q[0][e / 2] = (q[0][e / 2] & keep) | (0x7fffu << at);
+        q[1][e / 2] = (q[1][e / 2] & keep) | ((u >> 16) << at);
+        q[2][e / 2] = (q[2][e / 2] & keep) | ((u & 0xffffu) << at);
+      }
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < 3; ++p) out[p] = uint4{q[p][0], q[p][1], q[p][2], q[p][3]};
 }
+// A value from its parts (each in the upper half of a word).
+__device__ __forceinline__ float parts_value(uint32_t h, uint32_t m, uint32_t l) {
+  const float x = __uint_as_float(h);
+  return x == x ? (x + __uint_as_float(m)) + __uint_as_float(l) : __uint_as_float(m | l >> 16);
+}
+
 bool permute_w(const WPerm& pw);
 // Four filter re-layouts in one launch (null w: none).
 struct WPerm4 {

@@ -48,11 +48,13 @@ __device__ __forceinline__ void permute_w_elem(const WPerm& pw, uint32_t i) {
     out[i] = v;
     return;
   }
-  const Parts q = split_parts(v);
+  const Parts2 q = split_pair(v, 0.f);
+  const uint32_t u = __float_as_uint(v);
+  const bool raw = parts_raw(v);
   uint16_t* o = reinterpret_cast<uint16_t*>(out) + (size_t(r) * (ld / 16) + kk / 16) * 48 + kk % 16;
-  o[0] = uint16_t(q.h >> 16);
-  o[16] = uint16_t(q.m >> 16);
-  o[32] = uint16_t(q.l >> 16);
+  o[0] = uint16_t(raw ? 0x7fffu : q.h);
+  o[16] = uint16_t(raw ? u >> 16 : q.m);
+  o[32] = uint16_t(raw ? u : q.l);
 }
 
 __global__ void k_permute_w(WPerm pw) { permute_w_elem(pw, blockIdx.x * blockDim.x + threadIdx.x); }
@@ -108,9 +110,8 @@ struct BnDxArgs {
   float* dx;
   float eps, m;
 };
-// parts: the channel-innermost values also (or, with out null, only) as bf16
-// parts, [pixel][nblk][h, m, l of 16 channels]; a thread splits 8 channels of
-// a pixel and stores one 16-byte quad per part.
+// parts (CB = 32): the channel-innermost values also (or, with out null, only)
+// as bf16 parts, [pixel][nblk][h, m, l of 16 channels].
 template <int CB, bool BNDX = false>
 __global__ void __launch_bounds__(256)
     k_to_nhwc(const float* __restrict__ in, const float* __restrict__ y, float* __restrict__ out,
@@ -203,32 +204,35 @@ __global__ void __launch_bounds__(256)
     if (part == 0 && c0 + cl < C)
       dbPart[size_t(c0 + cl) * nB * npb + size_t(b) * npb + pb] = s;
   }
-  if (parts != nullptr) {
-    // Consecutive threads store consecutive quads: CB / 16 blocks of 6 per
-    // pixel, each thread splitting 8 channels for one part (that three
-    // threads split the same values costs less than 32-byte stores would).
-    constexpr int QB = CB / 16 * 6;
+  if constexpr (CB == 32) {
+    if (parts != nullptr) {
+      // A thread splits 8 channels of a pixel; the quads pass through LDS so
+      // that consecutive threads store consecutive ones (32-byte runs, which a
+      // thread's own quads would make, took longer).
+      constexpr int GP = CB / 8, QB = CB / 16 * 6;  // groups and quads of a pixel
+      static_assert(PB * GP == 256, "one group of 8 per thread");
+      __shared__ uint4 qs[PB * QB];
+      {
+        const int pl = tid / GP, gr = tid % GP;
+        float x[8];
 #pragma unroll
-    for (int j = 0; j < PB * QB / 256; ++j) {
-      const int s = tid + 256 * j, pl = s / QB, q = s - pl * QB, part = q % 6 / 2;
-      const int c8 = q / 6 * 16 + (q & 1) * 8;
-      const uint32_t p = p0 + pl;
-      if (p >= HW || c0 + c8 >= 16 * nblk) continue;
-      uint32_t u[8];
+        for (int e = 0; e < 8; ++e) x[e] = t[8 * gr + e][pl];
+        uint4 w[3];
+        split_parts8<false>(x, w);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const Parts a = split_parts(t[c8 + e][pl]);
-        u[e] = part == 0 ? a.h : part == 1 ? a.m : a.l;
+        for (int i = 0; i < 3; ++i) qs[pl * QB + gr / 2 * 6 + 2 * i + (gr & 1)] = w[i];
       }
-      uint4 v;
-      v.x = __builtin_amdgcn_perm(u[1], u[0], 0x07060302u);
-      v.y = __builtin_amdgcn_perm(u[3], u[2], 0x07060302u);
-      v.z = __builtin_amdgcn_perm(u[5], u[4], 0x07060302u);
-      v.w = __builtin_amdgcn_perm(u[7], u[6], 0x07060302u);
-      *reinterpret_cast<uint4*>(reinterpret_cast<char*>(parts) +
-                                ((size_t(b) * HW + p) * nblk + c0 / 16) * 96 + q * 16) = v;
+      __syncthreads();
+      const uint32_t qn = min(uint32_t(QB), 6 * (nblk - c0 / 16));  // quads inside the channels
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        const uint32_t s = tid + 256 * j, pl = s / QB, q = s - pl * QB, p = p0 + pl;
+        if (p < HW && q < qn)
+          *reinterpret_cast<uint4*>(reinterpret_cast<char*>(parts) +
+                                    ((size_t(b) * HW + p) * nblk + c0 / 16) * 96 + q * 16) = qs[s];
+      }
+      if (out == nullptr) return;
     }
-    if (out == nullptr) return;
   }
   const int cq = tid % (CB / 4);  // channel quad of the store phase
 #pragma unroll
@@ -881,6 +885,9 @@ bool packed_x(const ConvGeom& g) { return g.C < 4 && g.s > 4; }
 // -> 256 at 13 x 13, b128: 978 -> 824 us.
 bool conv_parts(const ConvGeom& g) {
   if (g.C < 32 || g.OC < 32) return false;
+  // dW over less than one 16-deep step gains nothing, and a sum of one product is
+  // the one that parts round worse (2.6e-8 against 2.5e-8).
+  if (g.B * g.OH * g.OW < 16) return false;
   if (double(g.k) * g.k * g.C * g.OC < 210.0 * (g.C + g.OC)) return false;
   return parts_floats(size_t(g.B) * g.H * g.W, g.C) < kOob &&
          parts_floats(size_t(g.B) * g.OH * g.OW, g.OC) < kOob &&

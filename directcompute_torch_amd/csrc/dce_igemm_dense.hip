@@ -124,12 +124,9 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 
   auto k_loop = [&](auto fp32) {
     constexpr bool FP32 = decltype(fp32)::value;
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+    f16v lo[FM][FN];
+    parts_zero(acc);
+    parts_zero(lo);
     typename LA::Regs ra[2];
     typename LB::Regs rb[2];
 #pragma unroll
@@ -155,7 +152,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
         for (int i = 0; i < FM; ++i) a[i][p] = SA::frag(Ac, p, wm * WM + 32 * i, lane);
       }
-      parts_mma<FP32>(a, b, acc);
+      parts_mma<FP32>(a, b, acc, lo);
       la.template store<!FP32>(ra[cur ^ 1], S + (cur ^ 1) * STAGE);
       lb.template store<!FP32>(rb[cur ^ 1], S + (cur ^ 1) * STAGE + SA::BYTES);
       __syncthreads();
@@ -164,6 +161,7 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
       step(kt, std::integral_constant<int, 0>{});
       if (kt + 1 < ke) step(kt + 1, std::integral_constant<int, 1>{});
     }
+    if constexpr (!FP32) parts_join(acc, lo);
   };
   k_loop(std::false_type{});
   if (__syncthreads_or(parts_bad(acc))) k_loop(std::true_type{});

@@ -3,21 +3,31 @@
 // linear layers' input gradient (dce_igemm_dense.hip).
 //
 // A float has a 24-bit significand and three bf16 have 3 x 8: x = h + m + l
-// exactly, each part the upper half of what the ones before it leave (exact
+// exactly, each part what the ones before it leave, rounded to nearest (exact
 // down to |x| = 8e-34, below which the last part's low bits leave the bf16
-// range).  Of the nine part products the six largest are kept; the dropped
-// m*l, l*m and l*l are below 2^-21 of the product.  gfx950 runs bf16 MFMAs at
-// 16 times the fp32 rate (1017 against 64 flops per cycle and SIMD), so six
-// of them take 3/8 of the fp32 MFMA's time.
+// range).  Of the nine part products the six largest are kept, as G. Henry,
+// P. T. P. Tang and A. Heinecke do ("Leveraging the bfloat16 artificial
+// intelligence datatype for higher-precision computations", 2019).  gfx950 runs
+// bf16 MFMAs at 16 times the fp32 rate (1017 against 64 flops per cycle and
+// SIMD), so six of them take 3/8 of the fp32 MFMA's time.
 //
-// The five smaller products of a 16-deep step are summed from zero and added
-// to the accumulator with an fp32 add, the largest goes into it directly.
-// That order is what keeps the result unbiased: a bf16 MFMA cuts its addends
-// off at the largest one's scale, always downwards, so with all six summed
-// together the 2^17 steps of a long dot product drift by 3e-7 of the result.
-// Error against float64 (2-norm, normal operands): 1.6e-7 at K = 576, 4.7e-7
-// at 4608 and 1.8e-6 at 65536, against 4.3e-7, 1.2e-6 and 4.6e-6 with
-// v_mfma_f32_16x16x4_f32.
+// Nearest, because |m| <= 2^-8 |x| and |l| <= 2^-17 |x| then have either sign:
+// the dropped m*l, l*m and l*l are at most 2^-24 of the product and average
+// out.  Cut-off parts drop up to 2^-21, always towards zero: 4e-8 of the result
+// at any length, and 2.4 times the fp32 error in sums of a few terms.
+//
+// The five smaller products have an accumulator of their own and the two are
+// added once, at the end.  The large one then sums 16-bit products, whose low
+// bits survive for many terms, and the small one's roundings are 2^-8 of the
+// result's.  A bf16 MFMA cuts its addends off at the largest one's scale, always
+// downwards: small products summed with the large ones drift by 3e-7 of the
+// result over 2^17 steps.
+//
+// Error against float64 (2-norm, normal operands), with v_mfma_f32_16x16x4_f32
+// and on parts: one product 2.5e-8 and 2.6e-8, 16 terms of 4096 6.3e-8 and
+// 5.8e-8, 576 terms 4.1e-7 and 7.9e-8, 4096 4.4e-7 and 1.5e-7, 25088 in splits
+// 2.1e-7 and 1.3e-7; gradients of which one value in 2000 survives a mask 5.6e-8
+// and 5.6e-8 (dW), 2.9e-8 and 2.6e-8 (dX).
 //
 // The operands are split once, by the pass that re-lays them out anyway, and
 // kept in memory as parts: the 16 channels of a block as 16 h, 16 m, 16 l (96
@@ -27,9 +37,10 @@
 // unit 37 % busy (64 -> 128 channels, 56 x 56: dW 433 us), with the split
 // before the LDS write and one LDS stage 476 us, with fp32 MFMAs 495 us.
 //
-// An operand that is infinite or NaN is kept as (h = x, 0, 0).  Such an
-// operand, or a product that overflows, leaves a NaN or an infinity in the
-// accumulator: that tile is computed again with fp32 MFMAs on x = h + m + l.
+// An operand without three finite bf16 parts (infinite, NaN, or so large that it
+// rounds to infinity) is kept as a NaN and its own two halves.  Such an operand,
+// or a product that overflows, leaves a NaN or an infinity in the accumulator:
+// that tile is computed again with fp32 MFMAs on the values themselves.
 //
 // The forward passes stay on fp32 MFMAs: their values decide ReLU masks and
 // max-pool routes, so another rounding there sends a few gradient elements of
@@ -350,48 +361,57 @@ struct PEpiPhase {
   }
 };
 
-// acc += a b for one 16-deep step: six bf16 products, or (FP32) the parts put
-// together again and multiplied in fp32.
+// hi + lo += a b for one 16-deep step: six bf16 products, or (FP32) the values put
+// together again and multiplied in fp32, into hi alone.
 template <bool FP32, int FM, int FN>
 __device__ __forceinline__ void parts_mma(const u4v (&a)[FM][3], const u4v (&b)[FN][3],
-                                          f16v (&acc)[FM][FN]) {
+                                          f16v (&hi)[FM][FN], f16v (&lo)[FM][FN]) {
   if constexpr (!FP32) {
+    auto product = [&](int pb, int pa, f16v (&acc)[FM][FN]) {
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      f16v t[FN];
+      for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j) t[j] = mfma_bf16(b[j][1], a[i][1], f16v{});
-#pragma unroll
-      for (int j = 0; j < FN; ++j) t[j] = mfma_bf16(b[j][0], a[i][2], t[j]);
-#pragma unroll
-      for (int j = 0; j < FN; ++j) t[j] = mfma_bf16(b[j][2], a[i][0], t[j]);
-#pragma unroll
-      for (int j = 0; j < FN; ++j) t[j] = mfma_bf16(b[j][0], a[i][1], t[j]);
-#pragma unroll
-      for (int j = 0; j < FN; ++j) t[j] = mfma_bf16(b[j][1], a[i][0], t[j]);
-#pragma unroll
-      for (int j = 0; j < FN; ++j) acc[i][j] = mfma_bf16(b[j][0], a[i][0], acc[i][j]);
-#pragma unroll
-      for (int j = 0; j < FN; ++j) acc[i][j] += t[j];
-    }
+        for (int j = 0; j < FN; ++j) acc[i][j] = mfma_bf16(b[j][pb], a[i][pa], acc[i][j]);
+    };
+    product(1, 1, lo);
+    product(0, 2, lo);
+    product(2, 0, lo);
+    product(0, 1, lo);
+    product(1, 0, lo);
+    product(0, 0, hi);
   } else {
     // Lane halves hold k = e and 8 + e: two k per fp32 MFMA.
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       auto word = [&](const u4v (&f)[3]) {
-        float x[3];
+        uint32_t x[3];
 #pragma unroll
-        for (int p = 0; p < 3; ++p)
-          x[p] = __uint_as_float(e & 1 ? f[p][e / 2] & 0xffff0000u : f[p][e / 2] << 16);
-        return (x[0] + x[1]) + x[2];
+        for (int p = 0; p < 3; ++p) x[p] = e & 1 ? f[p][e / 2] & 0xffff0000u : f[p][e / 2] << 16;
+        return parts_value(x[0], x[1], x[2]);
       };
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(word(b[j]), word(a[i]), acc[i][j], 0, 0, 0);
+          hi[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(word(b[j]), word(a[i]), hi[i][j], 0, 0, 0);
     }
   }
+}
+template <int FM, int FN>
+__device__ __forceinline__ void parts_zero(f16v (&acc)[FM][FN]) {
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+}
+template <int FM, int FN>
+__device__ __forceinline__ void parts_join(f16v (&hi)[FM][FN], const f16v (&lo)[FM][FN]) {
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) hi[i][j] += lo[i][j];
 }
 // Does the tile hold an infinity or a NaN?
 template <int FM, int FN>
@@ -454,12 +474,9 @@ __device__ __forceinline__ void gemm_parts_tile(char* S, const typename LA::Para
 
   auto k_loop = [&](auto fp32) {
     constexpr bool FP32 = decltype(fp32)::value;
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+    f16v lo[FM][FN];
+    parts_zero(acc);
+    parts_zero(lo);
     if (kb < ke) {
       la.issue(la, kb, S);
       lb.issue(lb, kb, S + SA::BYTES);
@@ -484,11 +501,12 @@ __device__ __forceinline__ void gemm_parts_tile(char* S, const typename LA::Para
         la.issue(la, kt + 1, S + (cur ^ 1) * STAGE);
         lb.issue(lb, kt + 1, S + (cur ^ 1) * STAGE + SA::BYTES);
       }
-      parts_mma<FP32>(a, b, acc);
+      parts_mma<FP32>(a, b, acc, lo);
       __builtin_amdgcn_sched_barrier(0);
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
     }
+    if constexpr (!FP32) parts_join(acc, lo);
   };
   k_loop(std::false_type{});
   if (__syncthreads_or(parts_bad(acc))) k_loop(std::true_type{});

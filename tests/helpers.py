@@ -46,3 +46,17 @@ def release(eng, *hs):
 
 def he(r, shape, fan_in):
     return (r.standard_normal(shape) * np.sqrt(2.0 / fan_in)).astype(np.float32)
+
+
+def fma_chain(a, b):
+    """A [M, K] by B [N, K] as a chain of fp32 FMAs along K."""
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    acc = np.zeros((a.shape[0], b.shape[0]), np.float32)
+    for k in range(a.shape[1]):
+        acc = (acc + np.outer(a[:, k], b[:, k])).astype(np.float32)
+    return acc
+
+
+def rel2(got, ref):
+    """2-norm of the difference over 2-norm of the result."""
+    return float(np.linalg.norm(np.asarray(got, np.float64) - ref) / np.linalg.norm(ref))

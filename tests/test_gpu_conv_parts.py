@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 
 from oracle import kernels as K
-from tests.helpers import download, he, release, rng, upload
+from tests.helpers import download, fma_chain, he, rel2, release, rng, upload
 
 pytestmark = pytest.mark.gpu
 
@@ -138,3 +138,44 @@ def test_special_values(eng, what):
             assert np.all(np.abs(a[fin] - b[fin]) <= 1e-5 * Sm + 1e-30)
         else:
             assert np.max(np.abs(a[fin] - b[fin])) <= tol * scale
+
+
+def _patches(a, k, p):
+    """[C][H][W] -> [pixels][(c, kh, kw)] of a stride-1 layer."""
+    C, H, W = a.shape
+    q = np.pad(a, ((0, 0), (p, p), (p, p)))
+    v = np.lib.stride_tricks.sliding_window_view(q, (k, k), (1, 2))
+    return np.ascontiguousarray(v.transpose(1, 2, 0, 3, 4).reshape(v.shape[1] * v.shape[2], -1))
+
+
+@pytest.mark.parametrize("keep", [0, 0.02, 0.25, 1], ids=["one", "2%", "25%", "dense"])
+def test_error_and_bias_against_fp32_fmas(eng, keep):
+    """Sums of one, few and many terms (a masked gradient) are no further from
+    float64 than a chain of fp32 FMAs, and not off to one side.  One term: 1.06,
+    its rounding and the dropped products."""
+    B, C, H, W, OC, k, s, p = 1, 64, 13, 13, 64, 3, 1, 1
+    r = rng(31)
+    x = r.standard_normal((B, C, H, W)).astype(np.float32)
+    w = he(r, (OC, C, k, k), C * k * k)
+    dy = r.standard_normal((B, OC, H, W)).astype(np.float32)
+    if keep == 0:
+        dy[:] = dy * (np.arange(H * W).reshape(H, W) == 85)
+    elif keep < 1:
+        dy *= r.random(dy.shape) < keep
+    dw, _, dx = _backward(eng, x, w, dy, None, s, p, 0)
+    ref = K.conv_backward(dy, dy, x, w, s, p, 0)
+    fdw = fma_chain(dy.reshape(OC, -1), _patches(x[0], k, p).T).reshape(w.shape)
+    flip = w[:, :, ::-1, ::-1].transpose(1, 0, 2, 3).reshape(C, -1)
+    fdx = fma_chain(flip, _patches(dy[0], k, k - 1 - p)).reshape(x.shape)
+    for name, got, want, fp32 in (("dW", dw, ref[0], fdw), ("dX", dx, ref[2], fdx)):
+        slack = 1.06 if name == "dW" and keep == 0 else 1.0
+        assert rel2(got, want) <= slack * rel2(fp32, want), name
+    # operands of one sign: nothing cancels a bias
+    dw, _, dx = _backward(eng, np.abs(x), np.abs(w), np.abs(dy), None, s, p, 0)
+    ref = K.conv_backward(np.abs(dy), dy, np.abs(x), np.abs(w), s, p, 0)
+    for name, got, want in (("dW", dw, ref[0]), ("dX", dx, ref[2])):
+        on = want > 0
+        err = (got[on] - want[on]) / want[on]
+        # 2^-28, a sixteenth of half a unit in the last place, and what a bf16 MFMA
+        # cuts off downwards: half of 2^-37 of the accumulator for each addend
+        assert abs(err.mean()) <= 2.0 ** -28 + OC * k * k * 2.0 ** -38, name

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 from oracle import kernels as K
-from tests.helpers import download, release, rng, upload
+from tests.helpers import download, fma_chain, rel2, release, rng, upload
 
 pytestmark = pytest.mark.gpu
 
@@ -63,3 +63,27 @@ def test_a_bt_not_finite(eng):
     assert np.array_equal(c[inf], ref[inf])
     fin = np.isfinite(ref)
     assert np.max(np.abs(c[fin] - ref[fin])) <= 1e-5 * np.max(np.abs(ref[fin]))
+
+
+@pytest.mark.parametrize("terms", [1, 4, 64, 4100])
+def test_a_bt_error_and_bias_against_fp32_fmas(eng, monkeypatch, terms):
+    """As for the convolutions: sums of few and many terms against a chain of fp32
+    FMAs (64 rows, 150 columns of the product); one term 1.06.  K is not split: the
+    sum of split partials rounds in either arithmetic."""
+    monkeypatch.setenv("DCE_TUNE_GEMM", "128,64,16,1")
+    M, Kd, N = 130, 4100, 3800
+    r = rng(terms)
+    a = r.standard_normal((M, Kd), dtype=np.float32)
+    b = r.standard_normal((N, Kd), dtype=np.float32)
+    if terms < Kd:
+        a *= np.stack([r.permutation(Kd) < terms for _ in range(M)])
+    part = np.s_[66:130, 3650:3800]
+    ref = a[part[0]].astype(np.float64) @ b[part[1]].T.astype(np.float64)
+    fp32 = rel2(fma_chain(a[part[0]], b[part[1]]), ref)
+    assert rel2(_matmul(eng, a, b)[part], ref) <= (1.06 if terms == 1 else 1.0) * fp32
+    a, b = np.abs(a), np.abs(b)
+    ref = a.astype(np.float64) @ b.T.astype(np.float64)
+    err = (_matmul(eng, a, b) - ref) / ref
+    # 2^-28, a sixteenth of half a unit in the last place, and what a bf16 MFMA cuts
+    # off downwards: half of 2^-37 of the accumulator for each of its 16 addends
+    assert abs(err.mean()) <= 2.0 ** -28 + terms * 2.0 ** -38
