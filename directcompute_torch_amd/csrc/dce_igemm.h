@@ -1820,13 +1820,19 @@ __device__ __forceinline__ Parts2 split_pair(float x, float y) {
   const uint32_t m = bf16_pair(rx, ry);
   return Parts2{h, m, bf16_pair(rx - __uint_as_float(m << 16), ry - __uint_as_float(m & 0xffff0000u))};
 }
-// x has no three finite bf16 parts: it is kept as a NaN, then its own upper and
-// lower half (parts_value puts it together again).
+// Below 2^-110 the last bits of a float leave the bf16 range, from 0x7f7f8000 on
+// it rounds to infinity: x has no three bf16 parts then.  It is kept as a NaN,
+// then its own upper and lower half (parts_value puts it together again).
+// `key` is the magnitude's bits, shifted so that zero, which has parts, is the
+// largest.
+__device__ __forceinline__ uint32_t parts_key(float x) { return (__float_as_uint(x) << 1) - 1u; }
+constexpr uint32_t kTinyKey = 2 * 0x08800000u - 1, kHugeKey = 2 * 0x7f7f8000u - 1;
 __device__ __forceinline__ bool parts_raw(float x) {
-  return (__float_as_uint(x) & 0x7fffffffu) >= 0x7f7f8000u;
+  const uint32_t k = parts_key(x);
+  return k < kTinyKey || (k >= kHugeKey && k != 0xffffffffu);
 }
-// Parts of 8 values as one 16-byte quad per part.  FINITE: nothing is raw (if
-// something is, it gets a NaN part).
+// Parts of 8 values as one 16-byte quad per part.  FINITE: nothing is raw (a
+// value at the upper end that is gets a NaN part).
 template <bool FINITE>
 __device__ __forceinline__ void split_parts8(const float (&x)[8], uint4 (&out)[3]) {
   uint32_t q[3][4];
@@ -1838,10 +1844,14 @@ __device__ __forceinline__ void split_parts8(const float (&x)[8], uint4 (&out)[3
     q[2][e] = p.l;
   }
   if constexpr (!FINITE) {
-    bool raw = false;
+    uint32_t least = 0xffffffffu, most = 0;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) raw |= parts_raw(x[e]);
-    if (raw) {  // hardly ever
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t k = parts_key(x[e]);
+      least = min(least, k);
+      most = max(most, k + 1u);
+    }
+    if (least < kTinyKey || most > kHugeKey) {  // hardly ever
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         if (!parts_raw(x[e])) continue;

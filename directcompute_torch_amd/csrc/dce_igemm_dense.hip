@@ -68,7 +68,8 @@ struct DSplit {
   static_assert(2 * R <= kThreads, "at most one group of 8 per thread");
   BRes b;
   uint32_t base, kd, k0;
-  int slot;  // of the h part; -1: none
+  int slot;        // of the h part; -1: none
+  uint32_t least;  // parts_key of the values stored as FINITE
   __device__ __forceinline__ void init(const Params& P, uint32_t row0, int t) {
     b.init(P.p, P.n);
     kd = P.kd;
@@ -76,6 +77,7 @@ struct DSplit {
     k0 = 8 * half;
     base = row < R && row0 + row < P.rows ? (row0 + row) * P.kd + k0 : kOob;
     slot = row < R ? row * 6 + (half ^ St::rhalf(row)) : -1;
+    least = 0xffffffffu;
   }
   __device__ __forceinline__ void load(uint32_t kt, uint32_t ke, Regs& r) const {
     const uint32_t k = kt * 16 + k0, o = base + kt * 16;
@@ -84,10 +86,13 @@ struct DSplit {
     r.v[1] = b.ld4(ok && k + 4 < kd ? o + 4 : kOob);
   }
   template <bool FINITE>
-  __device__ __forceinline__ void store(const Regs& r, char* S) const {
+  __device__ __forceinline__ void store(const Regs& r, char* S) {
     float x[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = r.v[e / 4][e % 4];
+    for (int e = 0; e < 8; ++e) {
+      x[e] = r.v[e / 4][e % 4];
+      if (FINITE) least = min(least, parts_key(x[e]));
+    }
     uint4 q[3];
     split_parts8<FINITE>(x, q);
     if (slot < 0) return;
@@ -164,7 +169,8 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
     if constexpr (!FP32) parts_join(acc, lo);
   };
   k_loop(std::false_type{});
-  if (__syncthreads_or(parts_bad(acc))) k_loop(std::true_type{});
+  if (__syncthreads_or(parts_bad(acc) || min(la.least, lb.least) < kTinyKey))
+    k_loop(std::true_type{});
   parts_store<PEpiRowMajor>(pe, acc, m0 + wm * WM, n0 + wn * WN, z, lane);
 }
 

@@ -3,13 +3,12 @@
 // linear layers' input gradient (dce_igemm_dense.hip).
 //
 // A float has a 24-bit significand and three bf16 have 3 x 8: x = h + m + l
-// exactly, each part what the ones before it leave, rounded to nearest (exact
-// down to |x| = 8e-34, below which the last part's low bits leave the bf16
-// range).  Of the nine part products the six largest are kept, as G. Henry,
-// P. T. P. Tang and A. Heinecke do ("Leveraging the bfloat16 artificial
-// intelligence datatype for higher-precision computations", 2019).  gfx950 runs
-// bf16 MFMAs at 16 times the fp32 rate (1017 against 64 flops per cycle and
-// SIMD), so six of them take 3/8 of the fp32 MFMA's time.
+// exactly, each part what the ones before it leave, rounded to nearest.  Of the
+// nine part products the six largest are kept, as G. Henry, P. T. P. Tang and A.
+// Heinecke do ("Leveraging the bfloat16 artificial intelligence datatype for
+// higher-precision computations", 2019).  gfx950 runs bf16 MFMAs at 16 times the
+// fp32 rate (1017 against 64 flops per cycle and SIMD), so six of them take 3/8
+// of the fp32 MFMA's time.
 //
 // Nearest, because |m| <= 2^-8 |x| and |l| <= 2^-17 |x| then have either sign:
 // the dropped m*l, l*m and l*l are at most 2^-24 of the product and average
@@ -37,10 +36,11 @@
 // unit 37 % busy (64 -> 128 channels, 56 x 56: dW 433 us), with the split
 // before the LDS write and one LDS stage 476 us, with fp32 MFMAs 495 us.
 //
-// An operand without three finite bf16 parts (infinite, NaN, or so large that it
-// rounds to infinity) is kept as a NaN and its own two halves.  Such an operand,
-// or a product that overflows, leaves a NaN or an infinity in the accumulator:
-// that tile is computed again with fp32 MFMAs on the values themselves.
+// An operand without three bf16 parts (infinite, NaN, so large that it rounds to
+// infinity, or not zero and below 2^-110 = 8e-34) is kept as a NaN and its own
+// two halves.  Such an operand, or a product that overflows, leaves a NaN or an
+// infinity in the accumulator: that tile is computed again with fp32 MFMAs on
+// the values themselves.
 //
 // The forward passes stay on fp32 MFMAs: their values decide ReLU masks and
 // max-pool routes, so another rounding there sends a few gradient elements of

@@ -100,11 +100,11 @@ def test_forced_tiles(eng, monkeypatch, tile):
         _check(_backward(eng, x, w, dy, y, s, p, act), x, w, dy, y, s, p, act)
 
 
-@pytest.mark.parametrize("what", ["inf", "nan", "quiet", "overflow", "tiny"])
+@pytest.mark.parametrize("what", ["inf", "nan", "quiet", "overflow", "tiny", "tiny weights", "few tiny", "denormal"])
 def test_special_values(eng, what):
     """Infinities and NaNs come out where IEEE arithmetic puts them (the tile is
-    computed again in fp32), and values whose last part leaves the bf16 range
-    lose no more than that."""
+    computed again in fp32), and so do values below the range of three bf16 parts,
+    to fp32's own bound: as many roundings of 2^-24, or 2^-149 below 2^-126."""
     case = (2, 64, 9, 10, 80, 3, 1, 1, 0)
     x, w, dy, y = _inputs(*case)
     s, p, act = case[6:]
@@ -116,8 +116,16 @@ def test_special_values(eng, what):
         dy[1, 60, 0, 0] = np.array([0x7F800001], np.uint32).view(np.float32)[0]
     elif what == "overflow":
         dy[0, 3, 2, 2], w[3, :, :, :] = 3e38, 3e5
-    else:
+    elif what == "tiny":
         dy *= np.float32(1e-36)
+    elif what == "tiny weights":
+        w *= np.float32(3e-35)
+    elif what == "few tiny":  # a channel alone: its sums have nothing larger in them
+        x[:, 9] *= np.float32(2e-37)
+        w[:, 9] *= np.float32(2e-37)
+        dy[:, 70] *= np.float32(2e-37)
+    else:
+        dy *= np.float32(1e-39)
     with np.errstate(all="ignore"):
         ref = K.conv_backward(dy, y, x, w, s, p, act)
     got = _backward(eng, x, w, dy, y, s, p, act)
@@ -130,9 +138,12 @@ def test_special_values(eng, what):
         assert np.array_equal(a[inf], b32[inf])
         fin = np.isfinite(b32)
         scale = np.max(np.abs(b[fin])) if what != "overflow" else np.maximum(np.abs(b[fin]), 1.0)
-        # tiny: operands of 1e-36 keep 16 bits (2^-15 of an operand at worst)
-        tol = 2.0 ** -14 if what == "tiny" else 1e-5
-        if what == "overflow":  # sums of huge terms cancel: relative to the sum of magnitudes
+        tol = 1e-5
+        if "tiny" in what or what == "denormal":
+            Sm = K.conv_backward(np.abs(dy), y, np.abs(x), np.abs(w), s, p, act)
+            Sm, n = (Sm[0], 180) if a is got[0] else (Sm[2], 720)
+            assert np.all(np.abs(a - b) <= (n + 256) * (2.0 ** -24 * Sm + 2.0 ** -149))
+        elif what == "overflow":  # sums of huge terms cancel: relative to the sum of magnitudes
             Sm = K.conv_backward(np.abs(dy), y, np.abs(x), np.abs(w), s, p, act)
             Sm = (Sm[0] if a is got[0] else Sm[2])[fin]
             assert np.all(np.abs(a[fin] - b[fin]) <= 1e-5 * Sm + 1e-30)

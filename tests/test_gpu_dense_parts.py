@@ -87,3 +87,24 @@ def test_a_bt_error_and_bias_against_fp32_fmas(eng, monkeypatch, terms):
     # 2^-28, a sixteenth of half a unit in the last place, and what a bf16 MFMA cuts
     # off downwards: half of 2^-37 of the accumulator for each of its 16 addends
     assert abs(err.mean()) <= 2.0 ** -28 + terms * 2.0 ** -38
+
+
+@pytest.mark.parametrize("scale", [1e-36, 1e-39, 1e-33])
+@pytest.mark.parametrize("which", ["a", "b", "row"])
+def test_a_bt_tiny(eng, which, scale):
+    """Values below the range of three bf16 parts (8e-34), and just above it: fp32's
+    bound, one rounding of 2^-24 or 2^-149 a term."""
+    M, Kd, N = 130, 4100, 3800
+    r = rng(17)
+    a = r.standard_normal((M, Kd), dtype=np.float32)
+    b = r.standard_normal((N, Kd), dtype=np.float32)
+    if which == "a":
+        a *= np.float32(scale)
+    elif which == "b":
+        b *= np.float32(scale)
+    else:
+        b[3799] *= np.float32(scale)
+    ref = a.astype(np.float64) @ b.T.astype(np.float64)
+    S = np.abs(a).astype(np.float64) @ np.abs(b).T.astype(np.float64)
+    # Kd roundings of random sign, each at most 2^-24 of a partial sum that S bounds
+    assert np.all(np.abs(_matmul(eng, a, b) - ref) <= 64 * 2.0 ** -24 * S + Kd * 2.0 ** -149)
