@@ -485,7 +485,7 @@ def _prof_all(lib):
             "gap_bwd", "upsample", "upsample_bwd", "dice_loss_grad", "bias_grad", "sgd", "adam",
             "grad_norm",
             "clip_scale", "relu", "relu6", "relu_grad", "relu6_grad", "sigmoid_grad", "grad_accum",
-            "slice", "conv_grad_nhwc", "nhwc")
+            "slice", "conv_grad_nhwc", "nhwc", "x_parts")
     out = {}
     for f in fams:
         n, ms, fl, by = ctypes.c_uint64(), ctypes.c_double(), ctypes.c_double(), ctypes.c_double()

@@ -110,16 +110,71 @@ struct BnDxArgs {
   float* dx;
   float eps, m;
 };
-// parts (CB = 32): the channel-innermost values also (or, with out null, only)
-// as bf16 parts, [pixel][nblk][h, m, l of 16 channels].
-template <int CB, bool BNDX = false>
+// A thread's parts of 8 channels, in the order of memory (quad i of group g =
+// threadIdx.x: block g / 2, part i, half g % 2), so that consecutive threads then
+// store consecutive quads (32-byte runs, which a thread's own quads would make,
+// took longer).
+__device__ __forceinline__ void stage_parts8(const float (&x)[8], uint4* qs) {
+  uint4 w[3];
+  split_parts8<false>(x, w);
+  const int gr = threadIdx.x;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) qs[gr / 2 * 6 + 2 * i + (gr & 1)] = w[i];
+  __syncthreads();
+}
+
+// The forward's channel-innermost copy of x as bf16 parts, 256 groups of 8
+// channels a workgroup.
+struct XSplit {
+  const float* src;  // null: no job
+  float* dst;
+  uint32_t groups, nblk, Cp;
+  FastDiv dGroups;  // of a pixel: 2 * nblk
+  uint32_t blocks() const { return src ? cdiv(groups, 256) : 0; }
+};
+__device__ __forceinline__ void xsplit_block(const XSplit& q, uint32_t blk, uint4* qs) {
+  const uint32_t g = blk * 256 + threadIdx.x, pix = fdiv(g, q.dGroups);
+  const uint32_t c = 8 * (g - pix * q.dGroups.d);
+  const float* src = q.src + size_t(pix) * q.Cp + c;
+  f4 v[2] = {zero4(), zero4()};
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    if (g < q.groups && c + 4 * i < q.Cp) v[i] = *reinterpret_cast<const f4*>(src + 4 * i);
+  const float x[8] = {v[0][0], v[0][1], v[0][2], v[0][3], v[1][0], v[1][1], v[1][2], v[1][3]};
+  stage_parts8(x, qs);
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const uint32_t s = threadIdx.x + 256 * j;
+    if (blk * 768 + s < 3 * q.groups)
+      reinterpret_cast<uint4*>(q.dst)[size_t(blk) * 768 + s] = qs[s];
+  }
+}
+__global__ void __launch_bounds__(256) k_xsplit(const XSplit q) {
+  __shared__ uint4 qs[768];
+  xsplit_block(q, blockIdx.x, qs);
+}
+static bool xsplit(const XSplit& q) {
+  ProfScope prof("x_parts", 0, 4.0 * double(q.groups) * 8 * 2.5);
+  hipLaunchKernelGGL(k_xsplit, dim3(q.blocks()), dim3(256), 0, stream(), q);
+  return check_launch("xsplit");
+}
+
+// PARTS (CB = 32): out as bf16 parts, [pixel][nblk][h, m, l of 16 channels]; the
+// workgroups past the filters' split a kept copy of x (xs).
+template <int CB, bool BNDX, bool PARTS>
 __global__ void __launch_bounds__(256)
     k_to_nhwc(const float* __restrict__ in, const float* __restrict__ y, float* __restrict__ out,
               float* __restrict__ dbPart, uint32_t C, uint32_t HW, uint32_t Cp, uint32_t npb,
-              uint32_t ncb, uint32_t nB, uint32_t nMain, WPerm pw, float* __restrict__ parts,
-              uint32_t nblk, BnDxArgs bn = BnDxArgs{}) {
+              uint32_t ncb, uint32_t nB, uint32_t nMain, WPerm pw, uint32_t nblk, uint32_t nPerm,
+              XSplit xs, BnDxArgs bn) {
+  static_assert(!PARTS || CB == 32, "parts: one group of 8 channels per thread");
+  __shared__ uint4 qs[PARTS ? 768 : 1];
   if (blockIdx.x >= nMain) {
-    permute_w_elem(pw, (blockIdx.x - nMain) * 256 + threadIdx.x);
+    const uint32_t e = blockIdx.x - nMain;
+    if (!PARTS || e < nPerm)
+      permute_w_elem(pw, e * 256 + threadIdx.x);
+    else
+      xsplit_block(xs, e - nPerm, qs);
     return;
   }
   constexpr int PB = 2048 / CB, PQ = PB / 4;  // pixels per block, pixel quads per row
@@ -204,35 +259,24 @@ __global__ void __launch_bounds__(256)
     if (part == 0 && c0 + cl < C)
       dbPart[size_t(c0 + cl) * nB * npb + size_t(b) * npb + pb] = s;
   }
-  if constexpr (CB == 32) {
-    if (parts != nullptr) {
-      // A thread splits 8 channels of a pixel; the quads pass through LDS so
-      // that consecutive threads store consecutive ones (32-byte runs, which a
-      // thread's own quads would make, took longer).
-      constexpr int GP = CB / 8, QB = CB / 16 * 6;  // groups and quads of a pixel
-      static_assert(PB * GP == 256, "one group of 8 per thread");
-      __shared__ uint4 qs[PB * QB];
-      {
-        const int pl = tid / GP, gr = tid % GP;
-        float x[8];
+  if constexpr (PARTS) {
+    constexpr int GP = CB / 8, QB = CB / 16 * 6;  // groups and quads of a pixel
+    {
+      const int pl = tid / GP, gr = tid % GP;
+      float x[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = t[8 * gr + e][pl];
-        uint4 w[3];
-        split_parts8<false>(x, w);
-#pragma unroll
-        for (int i = 0; i < 3; ++i) qs[pl * QB + gr / 2 * 6 + 2 * i + (gr & 1)] = w[i];
-      }
-      __syncthreads();
-      const uint32_t qn = min(uint32_t(QB), 6 * (nblk - c0 / 16));  // quads inside the channels
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const uint32_t s = tid + 256 * j, pl = s / QB, q = s - pl * QB, p = p0 + pl;
-        if (p < HW && q < qn)
-          *reinterpret_cast<uint4*>(reinterpret_cast<char*>(parts) +
-                                    ((size_t(b) * HW + p) * nblk + c0 / 16) * 96 + q * 16) = qs[s];
-      }
-      if (out == nullptr) return;
+      for (int e = 0; e < 8; ++e) x[e] = t[8 * gr + e][pl];
+      stage_parts8(x, qs);
     }
+    const uint32_t qn = min(uint32_t(QB), 6 * (nblk - c0 / 16));  // quads inside the channels
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const uint32_t s = tid + 256 * j, pl = s / QB, q = s - pl * QB, p = p0 + pl;
+      if (p < HW && q < qn)
+        *reinterpret_cast<uint4*>(reinterpret_cast<char*>(out) +
+                                  ((size_t(b) * HW + p) * nblk + c0 / 16) * 96 + q * 16) = qs[s];
+    }
+    return;
   }
   const int cq = tid % (CB / 4);  // channel quad of the store phase
 #pragma unroll
@@ -633,32 +677,36 @@ static uint32_t to_nhwc_rows(uint32_t B, uint32_t Cp, uint32_t HW) {
   return B * (Cp <= 16 ? cdiv(HW, 128) : cdiv(HW, 64));
 }
 
+// parts: out is bf16 parts (C > 16); xs rides in that launch.
 static bool to_nhwc_masked(const float* in, const float* y, float* out, float* dbPart,
                            uint32_t B, uint32_t C, uint32_t HW, uint32_t* npbOut,
-                           const WPerm& pw = WPerm{}, float* parts = nullptr) {
-  const uint32_t Cp = pad4(C);
+                           const WPerm& pw = WPerm{}, bool parts = false,
+                           const XSplit& xs = XSplit{}) {
+  const uint32_t Cp = pad4(C), nblk = pad16(C) / 16;
   // Family "conv_grad_nhwc": the masked dy -> G pass of the conv backward
   // (reads dy and y, writes G); "nhwc": a plain copy of an activation.
   ProfScope prof(y ? "conv_grad_nhwc" : "nhwc", 0,
-                 4.0 * double(B) * HW * ((y ? 2.0 : 1.0) * C + (out ? Cp : 0) + (parts ? 1.5 * pad16(C) : 0)));
-  if (Cp <= 8 && !y && !dbPart && !parts) {
+                 4.0 * double(B) * HW * ((y ? 2.0 : 1.0) * C + (parts ? 24 * nblk : Cp)) +
+                     4.0 * double(xs.groups) * 8 * 2.5);
+  if (Cp <= 8 && !y && !dbPart) {
     const uint32_t npix = B * HW;
     hipLaunchKernelGGL(k_to_nhwc_small, dim3(cdiv(npix, 256)), dim3(256), 0, stream(), in, out, C,
                        HW, Cp, npix, make_fastdiv(HW));
     return check_launch("to_nhwc") && (!pw.w || permute_w(pw));
   }
-  if (Cp <= 16) {
-    const uint32_t npb = cdiv(HW, 128), nMain = npb * B;
-    if (npbOut) *npbOut = npb;
-    hipLaunchKernelGGL(k_to_nhwc<16>, dim3(nMain + pw.blocks()), dim3(256), 0, stream(), in, y,
-                       out, dbPart, C, HW, Cp, npb, 1u, B, nMain, pw, parts, pad16(C) / 16);
-  } else {
-    const uint32_t npb = cdiv(HW, 64);
-    if (npbOut) *npbOut = npb;
-    const uint32_t ncb = cdiv(Cp, 32), nMain = npb * ncb * B;
-    hipLaunchKernelGGL(k_to_nhwc<32>, dim3(nMain + pw.blocks()), dim3(256), 0, stream(), in, y,
-                       out, dbPart, C, HW, Cp, npb, ncb, B, nMain, pw, parts, pad16(C) / 16);
-  }
+  const uint32_t npb = cdiv(HW, Cp <= 16 ? 128 : 64), ncb = Cp <= 16 ? 1 : cdiv(Cp, 32);
+  const uint32_t nMain = npb * ncb * B, nPerm = pw.blocks();
+  if (npbOut) *npbOut = npb;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nMain + nPerm + xs.blocks()), dim3(256), 0, stream(), in, y,
+                       out, dbPart, C, HW, Cp, npb, ncb, B, nMain, pw, nblk, nPerm, xs, BnDxArgs{});
+  };
+  if (parts)
+    go(k_to_nhwc<32, false, true>);
+  else if (Cp <= 16)
+    go(k_to_nhwc<16, false, false>);
+  else
+    go(k_to_nhwc<32, false, false>);
   return check_launch("to_nhwc");
 }
 
@@ -671,20 +719,21 @@ bool bn_dx_g(const float* x, const float* dy, const float* mean, const float* va
   const bool parts = layout == kGLayoutParts;
   if (uint64_t(B) * C * HW >= kOob || uint64_t(B) * HW * (parts ? 24 * nblk : Cp) >= kOob)
     return false;
-  float* gf = parts ? nullptr : g;
-  float* gq = parts ? g : nullptr;
   ProfScope prof("bn_bwd_dx", 0, 4.0 * double(B) * HW * (3.0 * C + (parts ? 24 * nblk : Cp)));
   const BnDxArgs bn{mean, var, gamma, dg, db, dx, eps, float(uint64_t(B) * HW)};
   // The same blocks (and bias partials) as the conv backward's transpose pass.
-  if (Cp <= 16) {
-    const uint32_t npb = cdiv(HW, 128), nMain = npb * B;
-    hipLaunchKernelGGL((k_to_nhwc<16, true>), dim3(nMain), dim3(256), 0, stream(), dy, x, gf,
-                       dbPart, C, HW, Cp, npb, 1u, B, nMain, WPerm{}, gq, nblk, bn);
-  } else {
-    const uint32_t npb = cdiv(HW, 64), ncb = cdiv(Cp, 32), nMain = npb * ncb * B;
-    hipLaunchKernelGGL((k_to_nhwc<32, true>), dim3(nMain), dim3(256), 0, stream(), dy, x, gf,
-                       dbPart, C, HW, Cp, npb, ncb, B, nMain, WPerm{}, gq, nblk, bn);
-  }
+  const uint32_t npb = cdiv(HW, Cp <= 16 ? 128 : 64), ncb = Cp <= 16 ? 1 : cdiv(Cp, 32);
+  const uint32_t nMain = npb * ncb * B;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nMain), dim3(256), 0, stream(), dy, x, g, dbPart, C, HW, Cp,
+                       npb, ncb, B, nMain, WPerm{}, nblk, 0u, XSplit{}, bn);
+  };
+  if (parts)
+    go(k_to_nhwc<32, true, true>);
+  else if (Cp <= 16)
+    go(k_to_nhwc<16, true, false>);
+  else
+    go(k_to_nhwc<32, true, false>);
   return check_launch("batchnorm_backward_dx");
 }
 
@@ -877,8 +926,8 @@ bool pw_x(const ConvGeom& g) {
 }
 bool packed_x(const ConvGeom& g) { return g.C < 4 && g.s > 4; }
 // Does the backward run on bf16 parts (dce_igemm_parts.h)?  The parts cost
-// traffic (x is kept as 6 bytes a value beside the forward's own copy, G
-// written and read as 6 instead of 4), which C * OC * k * k products per pixel
+// traffic (the forward's copy of x split to 6 bytes a value, G written and read
+// as 6 instead of 4), which C * OC * k * k products per pixel
 // have to pay for: 3 x 3 layers over 32 -> 32 and 32 -> 64 channels lose
 // (forward, passes and backward 136 -> 150 us at 8 x 128 x 128, 94 -> 108 us
 // at 8 x 64 x 64), 96 -> 32 and 64 -> 64 gain (303 -> 284, 133 -> 128 us), 384
@@ -911,24 +960,22 @@ PsGeom ps_geom(const ConvGeom& g) {
 size_t xcopy_floats(const ConvGeom& g) {
   if (pw_x(g)) return 4;  // no copy: a placeholder handle
   if (ps_x(g)) return ps_geom(g).floats;
-  if (conv_parts(g)) return parts_floats(size_t(g.B) * g.H * g.W, g.C);
   if (!packed_x(g)) return nhwc_floats(g.B, g.C, g.H, g.W);
   return size_t(g.B) * (g.H + 2 * g.p) * (g.W + 2 * g.p) * g.C;
 }
 
-// Floats of the copy of x the general conv path builds (a pointwise layer
-// that takes that path, for its ReLU mask, needs the NHWC copy its forward
-// did not keep).
+// Floats of the copy of x that the backward's general path reads: the kept one,
+// or one it builds (on parts always: the kept copy is the forward's, fp32, so
+// that a forward whose backward never comes pays nothing for it; a pointwise
+// layer that takes the general path, for its ReLU mask, has kept none).
 static size_t xbuild_floats(const ConvGeom& g) {
-  if (!pw_x(g)) return xcopy_floats(g);
-  return conv_parts(g) ? parts_floats(size_t(g.B) * g.H * g.W, g.C)
-                       : nhwc_floats(g.B, g.C, g.H, g.W);
+  if (conv_parts(g)) return parts_floats(size_t(g.B) * g.H * g.W, g.C);
+  return pw_x(g) ? nhwc_floats(g.B, g.C, g.H, g.W) : xcopy_floats(g);
 }
 
 uint32_t xcopy_tag(const ConvGeom& g) {
   if (pw_x(g)) return 0x40000u;
   if (ps_x(g)) return 0x20000u + g.p + (g.s << 8) + (g.k << 12);
-  if (conv_parts(g)) return 0x80000u;
   return packed_x(g) ? 0x10000u + g.p : pad4(g.C);
 }
 
@@ -1231,12 +1278,7 @@ bool conv_forward(const float* x, float* x_nhwc_keep, const float* w, const floa
   const bool pk = packed_x(g);
   const uint32_t Cp = pad4(g.C), KK = g.k * g.k, kdim = pk ? pad4(KK * g.C) : KK * Cp;
   const bool blk = !pk && blocked_k(Cp), s1 = g.s == 1;
-  // With a backward on bf16 parts the copy kept for it is x as parts, written
-  // by the same pass; the forward's own fp32 copy is then scratch.
-  const bool parts = conv_parts(g);
-  float* keepParts = parts ? x_nhwc_keep : nullptr;
-  if (parts) x_nhwc_keep = nullptr;
-  const size_t nx = parts ? nhwc_floats(g.B, g.C, g.H, g.W) : xcopy_floats(g);
+  const size_t nx = xcopy_floats(g);
   const uint32_t N = g.B * g.OH * g.OW;
   if (!operand_fits(nx, "conv_forward") || !operand_fits(size_t(g.OC) * kdim, "conv_forward"))
     return false;
@@ -1258,8 +1300,7 @@ bool conv_forward(const float* x, float* x_nhwc_keep, const float* w, const floa
   // The filter re-layout rides in the NHWC copy's launch.
   const WPerm fwdPerm{w, wp, g.OC, g.C, KK, pk ? g.C : Cp, kdim, 0, blk ? 1 : 0};
   if (pk ? !(to_pk(x, xn, g) && permute_w(fwdPerm))
-         : !to_nhwc_masked(x, nullptr, xn, nullptr, g.B, g.C, g.H * g.W, nullptr, fwdPerm,
-                            keepParts))
+         : !to_nhwc_masked(x, nullptr, xn, nullptr, g.B, g.C, g.H * g.W, nullptr, fwdPerm))
     return false;
   const double fl = 2.0 * g.OC * g.C * KK * double(g.B) * g.OH * g.OW;
   {
@@ -1467,7 +1508,7 @@ bool conv_backward(const float* dy, const float* y, const float* x, const float*
   const size_t nG = (useGnhwc && !preGn) ? al64(gFloats) : 0;
   const size_t nGp = (useGpad && !preG) ? al64(size_t(g.B) * g.OC * q.OHWp) : 0;
   const size_t nDb = (db && !preG && !preGn) ? al64(size_t(dbRows) * g.OC) : 0;
-  const size_t nX = (dw && !x_nhwc) ? al64(xbuild_floats(g)) : 0;
+  const size_t nX = (dw && (parts || !x_nhwc)) ? al64(xbuild_floats(g)) : 0;
   if (ps && !operand_fits(nGp, "conv_backward")) return false;
   TileCfg dwc{128, 128, 16, 1}, dxc{128, 128, 16, 1};
   size_t nP = 0, nW = 0, nQ = 0;
@@ -1531,11 +1572,18 @@ bool conv_backward(const float* dy, const float* y, const float* x, const float*
   // NHWC G), the bias-gradient sum in the dW finishing launch.
   const WPerm dxPerm{w, wt, g.OC, g.C, KK, OCp, KK * OCp, 1, dx && blocked_k(OCp) ? 1 : 0,
                      0, 0, 0, 0, 0, parts ? 1u : 0u};
+  // On parts the kept copy of x is split in that launch too, or by itself.
+  XSplit xsJob{};
+  if (dw && parts && x_nhwc) {
+    const uint32_t nblk = pad16(g.C) / 16;
+    xsJob = XSplit{x_nhwc, xs, g.B * HW * 2 * nblk, nblk, pad4(g.C), make_fastdiv(2 * nblk)};
+  }
   uint32_t npbGot = npb;
   if (useGnhwc && !preGn &&
-      !to_nhwc_masked(dy, y, parts ? nullptr : gn, useGpad ? nullptr : dbPart, g.B, g.OC, OHW,
-                      &npbGot, dx && !phased ? dxPerm : WPerm{}, parts ? gn : nullptr))
+      !to_nhwc_masked(dy, y, gn, useGpad ? nullptr : dbPart, g.B, g.OC, OHW, &npbGot,
+                      dx && !phased ? dxPerm : WPerm{}, parts, xsJob))
     return false;
+  if (preGn && xsJob.src && !xsplit(xsJob)) return false;
   // With the producer's G the dX filter re-layout rides in the dW finish
   // (which runs before dX), or runs by itself when no dW is asked for.
   const bool permInFinish = preGn && dx && !phased && dw;
@@ -1553,12 +1601,12 @@ bool conv_backward(const float* dy, const float* y, const float* x, const float*
     return conv_dx_gemm(dxc, wt, gn, dx, qpart, g, parts);
   };
   auto dw_gemm = [&]() {
-    const float* xn = x_nhwc;
+    const float* xn = xsJob.src ? xs : x_nhwc;
     if (!xn) {
       const bool built = ps ? to_ps(x, xs, g)
                          : pk ? to_pk(x, xs, g)
-                              : to_nhwc_masked(x, nullptr, parts ? nullptr : xs, nullptr, g.B, g.C,
-                                               HW, nullptr, WPerm{}, parts ? xs : nullptr);
+                              : to_nhwc_masked(x, nullptr, xs, nullptr, g.B, g.C, HW, nullptr,
+                                               WPerm{}, parts);
       if (!built) return false;
       xn = xs;
     }

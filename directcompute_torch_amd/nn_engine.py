@@ -1385,7 +1385,7 @@ class KernelProfiler:
 
     # Families the engine records: the fused paths and every RunShader
     # kernel that runs under its own name.
-    FAMILIES = ("conv_fwd", "conv_bwd", "conv_dw", "conv_dx", "gemm", "nhwc", "conv_grad_nhwc",
+    FAMILIES = ("conv_fwd", "conv_bwd", "conv_dw", "conv_dx", "gemm", "nhwc", "conv_grad_nhwc", "x_parts",
                 "maxpool_fwd", "maxpool_bwd", "bn_stats", "bn_stats_side", "bn_fwd", "bn_bwd_reduce",
                 "bn_bwd_reduce_side", "bn_bwd_dx",
                 "dw_bwd_input", "dw_bwd_filter", "gap_bwd", "upsample", "upsample_bwd", "bias_grad",

@@ -190,3 +190,51 @@ def test_error_and_bias_against_fp32_fmas(eng, keep):
         # 2^-28, a sixteenth of half a unit in the last place, and what a bf16 MFMA
         # cuts off downwards: half of 2^-37 of the accumulator for each addend
         assert abs(err.mean()) <= 2.0 ** -28 + OC * k * k * 2.0 ** -38, name
+
+
+def _bytes(eng, fam):
+    n, v = ctypes.c_uint64(), [ctypes.c_double() for _ in range(3)]
+    ok = eng.lib.GetProfile(fam.encode(), ctypes.byref(n), *[ctypes.byref(d) for d in v])
+    return v[2].value if ok else 0.0
+
+
+def test_forward_alone_pays_nothing(eng):
+    """A forward that may get a backward moves and holds what one without does: its
+    own fp32 copy of x (33 channels: 36 in memory, 48 as parts).  The backward
+    splits that copy, and only for a dW."""
+    B, C, H, W, OC, k, s, p, act = CASES[4]
+    x, w, dy, y = _inputs(*CASES[4])
+    hx, hw, hb = upload(eng, x), upload(eng, w), upload(eng, np.zeros(OC, np.float32))
+    hdy = upload(eng, dy)
+    eng.lib.SetProfiling(1)
+    try:
+        moved = []
+        for pim in (None, ctypes.c_void_p()):
+            eng.lib.ResetProfile()
+            hy = eng.lib.ConvForwardFused(hx, hw, hb, B, C, H, W, OC, k, k, s, p, 0,
+                                          None if pim is None else ctypes.byref(pim))
+            assert hy, eng.last_error()
+            moved.append(_bytes(eng, "nhwc"))
+            release(eng, hy)
+        assert moved[0] == moved[1] == 4.0 * B * H * W * (C + 36)
+        # dX alone (frozen filters)
+        eng.lib.ResetProfile()
+        pdx = ctypes.c_void_p()
+        eng.lib.ConvBackwardFused(hdy, None, hx, hw, pim.value, B, C, H, W, OC, k, k, s, p, 0, 1, 0, 0,
+                                  None, None, ctypes.byref(pdx))
+        assert pdx.value, eng.last_error()
+        assert _bytes(eng, "x_parts") == 0 and _bytes(eng, "nhwc") == 4.0 * (dy.size + dy.size // OC * 144 * 1.5)
+        release(eng, pdx.value)
+    finally:
+        eng.lib.SetProfiling(0)
+        eng.lib.ResetProfile()
+    # what a handle holds: the pool gets it back when it is released
+    eng.lib.DrainPool()
+    pim = ctypes.c_void_p()
+    hy = eng.lib.ConvForwardFused(hx, hw, hb, B, C, H, W, OC, k, k, s, p, 0, ctypes.byref(pim))
+    assert hy and pim.value, eng.last_error()
+    before = eng.lib.GetPoolMemory()
+    release(eng, pim.value)
+    held = eng.lib.GetPoolMemory() - before
+    assert 4 * B * H * W * 36 <= held < 1.2 * 4 * B * H * W * 36, held
+    release(eng, hx, hw, hb, hdy, hy)
