@@ -425,7 +425,7 @@ struct LdNchwRK : LoaderBase<Stage<R, KT, false>> {
 //        oh*s == a + p - kh exactly (S1: s == 1, no divisibility test).
 //        A strided dX runs as s*s sub-pixel phases, each an S1 gather over
 //        its own grid of input pixels with nh x nw taps (k = nw) and the
-//        column origin shifted by pwd (conv_dx_phased).
+//        column origin shifted by pwd (conv_dx_plan).
 // ---------------------------------------------------------------------------
 constexpr int kCB = 16;
 
@@ -1898,11 +1898,14 @@ TileCfg conv_dw_choose(uint32_t M, uint32_t N, uint32_t kdim, bool trans, bool p
                        bool parts);
 bool conv_dw_gemm(const TileCfg& c, const float* gn, const float* xn, float* part,
                   const ConvGeom& g, bool trans, bool pk, bool ps, bool parts);
-TileCfg conv_dx_choose(const ConvGeom& g, bool parts);
-bool conv_dx_gemm(const TileCfg& c, const float* wt, const float* gn, float* dx, float* part,
-                  const ConvGeom& g, bool parts);
-bool conv_dx_phased(const float* w, float* wt, const float* gn, float* dx, const ConvGeom& g,
-                    bool parts);
+struct DxPlan {
+  bool phased;   // as sub-pixel phases, which re-lay the filters themselves (w -> wt)
+  TileCfg cfg;   // of the one launch (stride 3 or more: chosen per phase)
+  size_t part;   // floats of split partials
+};
+DxPlan conv_dx_plan(const ConvGeom& g, bool parts);
+bool conv_dx(const DxPlan& p, const float* w, float* wt, const float* gn, float* dx, float* part,
+             const ConvGeom& g, bool parts);
 
 // K order: blocked when the padded channel count is a multiple of kCB (no
 // extra padding then), flat otherwise.

@@ -937,7 +937,15 @@ bool conv_parts(const ConvGeom& g) {
   // dW over less than one 16-deep step gains nothing, and a sum of one product is
   // the one that parts round worse (2.6e-8 against 2.5e-8).
   if (g.B * g.OH * g.OW < 16) return false;
-  if (double(g.k) * g.k * g.C * g.OC < 210.0 * (g.C + g.OC)) return false;
+  const double products = double(g.k) * g.k * g.C * g.OC, x = double(g.B) * g.C * g.H * g.W;
+  if (products < 210.0 * (g.C + g.OC)) return false;
+  // At stride 3 and more an output pixel stands for s * s pixels of x.  Where
+  // their parts are real traffic they have to be paid for too (118 x 289 x 15 x
+  // 108 -> 88, k3 s4 583 on fp32, 649 us on parts; 53 x 56 x 93 x 94 -> 510, k3
+  // s4 687 and 751); smaller layers are bound by launches and latency and gain
+  // 9 % over 96 shapes (from -43 to +6 %).
+  if (g.s >= 3 && x >= 1e7 && products < 210.0 * (x / (double(g.B) * g.OH * g.OW) + g.OC))
+    return false;
   return parts_floats(size_t(g.B) * g.H * g.W, g.C) < kOob &&
          parts_floats(size_t(g.B) * g.OH * g.OW, g.OC) < kOob &&
          parts_floats(size_t(g.C) * g.k * g.k, g.OC) < kOob;
@@ -1510,7 +1518,7 @@ bool conv_backward(const float* dy, const float* y, const float* x, const float*
   const size_t nDb = (db && !preG && !preGn) ? al64(size_t(dbRows) * g.OC) : 0;
   const size_t nX = (dw && (parts || !x_nhwc)) ? al64(xbuild_floats(g)) : 0;
   if (ps && !operand_fits(nGp, "conv_backward")) return false;
-  TileCfg dwc{128, 128, 16, 1}, dxc{128, 128, 16, 1};
+  TileCfg dwc{128, 128, 16, 1};
   size_t nP = 0, nW = 0, nQ = 0;
   bool dwT = false;
   if (dw) {
@@ -1522,27 +1530,10 @@ bool conv_backward(const float* dy, const float* y, const float* x, const float*
     dwc = conv_dw_choose(dM, dN, dwK, dwT, pk, ps, parts);
     nP = al64(size_t(dwc.splits) * 4 * cdiv(size_t(g.OC) * taps, 4));
   }
-  // A dX at stride 3 or more runs as sub-pixel phases (conv_dx_phased), each with
-  // its own filter re-layout and no split: the strided gather would walk
-  // s^2 times the taps that reach a pixel (AlexNet c1's dX at b128: 18.0 ->
-  // 1.24 ms).  At stride 2 the four phases share one launch.  On parts they are
-  // always taken (12 x 37 x 61 x 45 -> 70, k5: dX 78 -> 32 us).  On fp32 MFMAs
-  // (forward and backward, gather -> phases; B x C x H x W -> OC): 128 x 8 x
-  // 100 x 90 -> 40, k3 338 -> 229, 32 x 16 x 112 x 112 -> 24, k3 102 -> 85, 20
-  // x 160 x 160 -> 31, k5 75 -> 58, 64 x 128 x 28 x 28 -> 256, k1 104 -> 84 us.
-  // Not where the gather splits its k * k taps so often that the largest
-  // phase's unsplit taps, (k + 1) / 2 squared, make the longer chain (30 x 9 x
-  // 9 -> 384, k5 79 -> 131, 128 x 30 x 7 x 7 -> 384, k5 149 -> 180 us), nor
-  // where the products saved do not pay for the launches added, the filters'
-  // and for k = 1 the zeros' (8 x 16 x 64 x 64 -> 24, k3 37 -> 41, 16 x 64 x
-  // 56 x 56 -> 128, k1 alone 76 -> 88 us).
-  bool phased = dx && (g.s >= 3 || (parts && g.s == 2));
-  if (dx && !phased) {
-    dxc = conv_dx_choose(g, parts);
-    const uint32_t kp = (g.k + 1) / 2;
-    const double products = double(g.C) * g.B * HW * KK * OCp;
-    phased = g.s == 2 && dxc.splits * kp * kp <= KK && products >= (g.k == 1 ? 8e8 : 2e8);
-    if (!phased) nQ = dxc.splits > 1 ? size_t(dxc.splits) * g.C * g.B * HW : 0;
+  DxPlan dxp{};
+  if (dx) {
+    dxp = conv_dx_plan(g, parts);
+    nQ = dxp.part;
   }
   if (dx) nW = al64(wFloats);
   float* ws = workspace(nG + nGp + nDb + nX + nP + nW + nQ);
@@ -1581,13 +1572,13 @@ bool conv_backward(const float* dy, const float* y, const float* x, const float*
   uint32_t npbGot = npb;
   if (useGnhwc && !preGn &&
       !to_nhwc_masked(dy, y, gn, useGpad ? nullptr : dbPart, g.B, g.OC, OHW, &npbGot,
-                      dx && !phased ? dxPerm : WPerm{}, parts, xsJob))
+                      dx && !dxp.phased ? dxPerm : WPerm{}, parts, xsJob))
     return false;
   if (preGn && xsJob.src && !xsplit(xsJob)) return false;
   // With the producer's G the dX filter re-layout rides in the dW finish
   // (which runs before dX), or runs by itself when no dW is asked for.
-  const bool permInFinish = preGn && dx && !phased && dw;
-  if (preGn && dx && !phased && !dw && !permute_w(dxPerm)) return false;
+  const bool permInFinish = preGn && dx && !dxp.phased && dw;
+  if (preGn && dx && !dxp.phased && !dw && !permute_w(dxPerm)) return false;
   const uint32_t dbRowsGot =
       (preG || preGn) ? pre->dbRows : (useGpad ? dbRows : g.B * npbGot);
   if (db && !dw) {
@@ -1597,8 +1588,7 @@ bool conv_backward(const float* dy, const float* y, const float* x, const float*
   auto dx_chain = [&]() {
     ProfScope prof("conv_dx", 2.0 * g.OC * g.C * KK * double(npix),
                    4.0 * (double(npix) * OCp + double(g.B) * g.C * g.H * g.W));
-    if (phased) return conv_dx_phased(w, wt, gn, dx, g, parts);
-    return conv_dx_gemm(dxc, wt, gn, dx, qpart, g, parts);
+    return conv_dx(dxp, w, wt, gn, dx, qpart, g, parts);
   };
   auto dw_gemm = [&]() {
     const float* xn = xsJob.src ? xs : x_nhwc;

@@ -134,14 +134,46 @@ struct DxPartsRun {
   }
 };
 
+static PhaseGeom phase_geom(const ConvGeom& g, uint32_t ph, uint32_t pw) {
+  const uint32_t s = g.s;
+  PhaseGeom q{};
+  q.ph = ph;
+  q.pw = pw;
+  q.GH = ph < g.H ? cdiv(g.H - ph, s) : 0;
+  q.GW = pw < g.W ? cdiv(g.W - pw, s) : 0;
+  q.rh = (ph + g.p) % s;
+  q.rw = (pw + g.p) % s;
+  q.nh = q.rh < g.k ? cdiv(g.k - q.rh, s) : 0;
+  q.nw = q.rw < g.k ? cdiv(g.k - q.rw, s) : 0;
+  q.qh = (ph + g.p - q.rh) / s;
+  q.qw = (pw + g.p - q.rw) / s;
+  return q;
+}
+
 // The phases of a stride-2 dX that some tap reaches, in one launch.
 struct DxPhases {
-  const float* gn;
-  float* dx;
   ConvGeom g;
   PhaseGeom q[4];
+  uint32_t n, cols, kmax;  // phases, their pixels together, the longest dot product
+  bool empty;              // pixels that no tap reaches
+  const float* gn;
+  float* dx;
   const float* wt[4];
-  uint32_t n;
+  uint32_t splits;
+  float* part;  // splits > 1: partials, each laid out as dx
+  DxPhases(const ConvGeom& geom, bool parts) : g(geom), n(0), cols(0), kmax(0), empty(false) {
+    for (uint32_t i = 0; i < 4; ++i) {
+      const PhaseGeom f = phase_geom(g, i / 2, i % 2);
+      if (f.GH * f.GW == 0) continue;
+      if (f.nh * f.nw == 0) {
+        empty = true;
+        continue;
+      }
+      q[n++] = f;
+      cols += g.B * f.GH * f.GW;
+      kmax = std::max(kmax, f.nh * f.nw * (parts ? pad16(g.OC) : pad4(g.OC)));
+    }
+  }
   // f(i, phase, columns) fills product i; returns the workgroups of them all.
   template <class A, class F>
   uint32_t fill(A& a, uint32_t MT, uint32_t NT, F&& f) const {
@@ -158,6 +190,7 @@ struct DxPhases {
   }
 };
 struct DxMultiParts : DxPhases {
+  using DxPhases::DxPhases;
   using EPI = PEpiPhase;
   template <int MT, int NT>
   int occ(bool) const {
@@ -174,15 +207,19 @@ struct DxMultiParts : DxPhases {
       a.pb[i] = {gn, g.OH, g.OW, no, f.nw, 1, f.qh, f.GW, GHW, N,
                  uint32_t(parts_floats(size_t(g.B) * g.OH * g.OW, g.OC)), make_fastdiv(GHW),
                  make_fastdiv(f.GW), make_fastdiv(KK), make_fastdiv(f.nw), int(f.qw) - int(f.qh)};
-      a.pe[i] = {dx, g.C, g.H, g.W, f.GW, GHW, N, g.s, f.ph, f.pw, a.pb[i].dGridHW, a.pb[i].dGridW};
+      a.pe[i] = {splits > 1 ? part : dx, g.C,  g.H,  g.W,  f.GW, GHW, N, g.s, f.ph, f.pw,
+                 a.pb[i].dGridHW,        a.pb[i].dGridW};
     });
-    hipLaunchKernelGGL((k_gemm_parts_multi<MT, NT, PRows<MT>, PPix<NT, true>, EPI>), dim3(wgs),
-                       dim3(kThreads), 0, stream(), a);
-    return check_launch("conv_backward_input");
+    const uint32_t values = g.B * g.C * g.H * g.W;
+    hipLaunchKernelGGL((k_gemm_parts_multi<MT, NT, PRows<MT>, PPix<NT, true>, EPI>),
+                       dim3(wgs * splits), dim3(kThreads), 0, stream(), a, wgs, splits, values);
+    return check_launch("conv_backward_input") &&
+           (splits == 1 || split_sum(part, dx, values, splits));
   }
 };
 template <bool BLK>
 struct DxMulti : DxPhases {
+  using DxPhases::DxPhases;
   template <int MT, int NT, int KT>
   int occ(bool) const {
     return occupancy(k_igemm_multi<MT, NT, KT, LdDenseRK<MT, KT>, LdPixRK<NT, KT, false, true, BLK>,
@@ -204,52 +241,32 @@ struct DxMulti : DxPhases {
 };
 // Their filters are re-laid by one launch too; phases that no tap reaches (k =
 // 1) are zero.
-template <class Geom>
-static bool phases_in_one(const float* w, float* wt, const float* gn, float* dx, const ConvGeom& g,
-                          bool parts, Geom&& geom) {
+template <class R>
+static bool phases_in_one(R& r, const TileCfg& c, const float* w, float* wt, const float* gn,
+                          float* dx, float* part, bool parts) {
+  const ConvGeom& g = r.g;
   const uint32_t OCp = parts ? pad16(g.OC) : pad4(g.OC);
-  const bool blk = blocked_k(OCp);
-  DxPhases m{};
-  m.gn = gn;
-  m.dx = dx;
-  m.g = g;
   WPerm4 pw{};
-  uint32_t cols = 0, kmax = 0;
-  bool empty = false;
   float* at = wt;
-  for (uint32_t i = 0; i < 4; ++i) {
-    const PhaseGeom q = geom(i / 2, i % 2);
+  for (uint32_t i = 0; i < r.n; ++i) {
+    const PhaseGeom& q = r.q[i];
     const uint32_t KK = q.nh * q.nw;
-    if (q.GH * q.GW == 0) continue;
-    if (KK == 0) {
-      empty = true;
-      continue;
-    }
-    pw.p[m.n] = WPerm{w, at, g.OC, g.C, KK, OCp, KK * OCp, 1, blk ? 1 : 0, q.nw, g.k, 2, q.rh, q.rw,
-                      parts ? 1u : 0u};
-    m.wt[m.n] = at;
-    m.q[m.n++] = q;
+    pw.p[i] = WPerm{w, at, g.OC, g.C, KK, OCp, KK * OCp, 1, blocked_k(OCp) ? 1 : 0, q.nw, g.k, 2,
+                    q.rh, q.rw, parts ? 1u : 0u};
+    r.wt[i] = at;
     at += parts ? parts_floats(size_t(g.C) * KK, g.OC) : size_t(g.C) * KK * OCp;
-    cols += g.B * q.GH * q.GW;
-    kmax = std::max(kmax, KK * OCp);
   }
-  if (empty && !fill_zero(dx, size_t(g.B) * g.C * g.H * g.W)) return false;
-  if (m.n == 0) return true;
+  r.gn = gn;
+  r.dx = dx;
+  r.splits = c.splits;
+  r.part = part;
+  if (r.empty && !fill_zero(dx, size_t(g.B) * g.C * g.H * g.W)) return false;
+  if (r.n == 0) return true;
   if (!permute_w4(pw)) return false;
-  if (parts) {
-    const DxMultiParts r{m};
-    const TileCfg t = parts_choose("DCE_TUNE_DX", g.C, cols, kmax, 1, true,
-                                   [&](const TileCfg& v) { return parts_occ(v, r); });
-    return parts_dispatch(t, r);
-  }
-  auto go = [&](const auto& r) {
-    TileCfg c = choose("DCE_TUNE_DX", g.C, cols, kmax, 1, true,
-                       [&](const TileCfg& t) { return tiles_occ16(t, r); }, true);
-    narrow_short_k(c, "DCE_TUNE_DX", g.C, cols, kmax);
-    c.splits = 1;
+  if constexpr (std::is_same<R, DxMultiParts>::value)
+    return parts_dispatch(c, r);
+  else
     return tiles_dispatch16(c, r);
-  };
-  return blk ? go(DxMulti<true>{m}) : go(DxMulti<false>{m});
 }
 
 // dX of a strided convolution as its s*s sub-pixel phases: every input pixel
@@ -257,35 +274,20 @@ static bool phases_in_one(const float* w, float* wt, const float* gn, float* dx,
 // k*k taps for every pixel and finds all but about 1/s^2 of them out of
 // step.  Each phase gets its own filter re-layout (into wt, C * k*k * OCp
 // floats) and GEMM, unsplit; phases that no tap reaches (k < s) are zero.
-bool conv_dx_phased(const float* w, float* wt, const float* gn, float* dx, const ConvGeom& g,
-                    bool parts) {
+static bool dx_phases(const float* w, float* wt, const float* gn, float* dx, const ConvGeom& g,
+                      bool parts) {
   const uint32_t s = g.s, OCp = parts ? pad16(g.OC) : pad4(g.OC);
   const bool blk = blocked_k(OCp);
-  auto geom = [&](uint32_t ph, uint32_t pw) {
-    PhaseGeom q{};
-    q.ph = ph;
-    q.pw = pw;
-    q.GH = ph < g.H ? cdiv(g.H - ph, s) : 0;
-    q.GW = pw < g.W ? cdiv(g.W - pw, s) : 0;
-    q.rh = (ph + g.p) % s;
-    q.rw = (pw + g.p) % s;
-    q.nh = q.rh < g.k ? cdiv(g.k - q.rh, s) : 0;
-    q.nw = q.rw < g.k ? cdiv(g.k - q.rw, s) : 0;
-    q.qh = (ph + g.p - q.rh) / s;
-    q.qw = (pw + g.p - q.rw) / s;
-    return q;
-  };
-  if (s == 2) return phases_in_one(w, wt, gn, dx, g, parts, geom);
   bool empty = false;
   for (uint32_t ph = 0; ph < s; ++ph)
     for (uint32_t pw = 0; pw < s; ++pw) {
-      const PhaseGeom q = geom(ph, pw);
+      const PhaseGeom q = phase_geom(g, ph, pw);
       empty |= q.GH * q.GW > 0 && q.nh * q.nw == 0;
     }
   if (empty && !fill_zero(dx, size_t(g.B) * g.C * g.H * g.W)) return false;
   for (uint32_t ph = 0; ph < s; ++ph)
     for (uint32_t pw = 0; pw < s; ++pw) {
-      const PhaseGeom q = geom(ph, pw);
+      const PhaseGeom q = phase_geom(g, ph, pw);
       if (q.GH * q.GW == 0 || q.nh * q.nw == 0) continue;
       const uint32_t KK = q.nh * q.nw, kdim = KK * OCp, N = g.B * q.GH * q.GW;
       if (!permute_w(WPerm{w, wt, g.OC, g.C, KK, OCp, kdim, 1, blk ? 1 : 0, q.nw, g.k, s, q.rh,
@@ -313,8 +315,8 @@ bool conv_dx_phased(const float* w, float* wt, const float* gn, float* dx, const
   return true;
 }
 
-
-TileCfg conv_dx_choose(const ConvGeom& g, bool parts) {
+// The whole gather.
+static TileCfg dx_choose(const ConvGeom& g, bool parts) {
   const uint32_t N = g.B * g.H * g.W;
   const bool s1 = g.s == 1;
   if (parts)
@@ -331,13 +333,70 @@ TileCfg conv_dx_choose(const ConvGeom& g, bool parts) {
   narrow_short_k(c, "DCE_TUNE_DX", g.C, N, kdim);
   return c;
 }
-bool conv_dx_gemm(const TileCfg& c, const float* wt, const float* gn, float* dx, float* part,
-                  const ConvGeom& g, bool parts) {
+// All phases of a stride-2 dX.
+static TileCfg dx_choose_phases(const ConvGeom& g, bool parts) {
+  if (parts) {
+    const DxMultiParts r(g, true);
+    return parts_choose("DCE_TUNE_DX", g.C, r.cols, r.kmax, r.empty ? 1 : 8, true,
+                        [&](const TileCfg& v) { return parts_occ(v, r); });
+  }
+  const DxPhases r(g, false);
+  auto go = [&](const auto& run) {
+    TileCfg c = choose("DCE_TUNE_DX", g.C, r.cols, r.kmax, 1, true,
+                       [&](const TileCfg& t) { return tiles_occ16(t, run); }, true);
+    narrow_short_k(c, "DCE_TUNE_DX", g.C, r.cols, r.kmax);
+    c.splits = 1;
+    return c;
+  };
+  return blocked_k(pad4(g.OC)) ? go(DxMulti<true>(g, false)) : go(DxMulti<false>(g, false));
+}
+
+// How a dX runs.  At stride 3 or more as sub-pixel phases (dx_phases), each with
+// its own filter re-layout and no split: the strided gather would walk s^2 times
+// the taps that reach a pixel (AlexNet c1's dX at b128: 18.0 -> 1.24 ms).  At
+// stride 2 the four phases share one launch.  On parts they are always taken (12
+// x 37 x 61 x 45 -> 70, k5: dX 78 -> 32 us), split where few pixels meet long dot
+// products (forward and backward, gather on fp32 MFMAs, unsplit and split
+// phases: 7 x 137 x 6 x 7 -> 505, k3 65, 97 and 56, 1 x 56 x 7 x 31 -> 384, k7
+// 175, 211 and 80, 32 x 39 x 6 x 10 -> 287, k3 60, 78 and 52 us).  On fp32 MFMAs they are unsplit (forward and backward, gather ->
+// phases; B x C x H x W -> OC): 128 x 8 x 100 x 90 -> 40, k3 338 -> 229, 32 x 16
+// x 112 x 112 -> 24, k3 102 -> 85, 20 x 160 x 160 -> 31, k5 75 -> 58, 64 x 128 x
+// 28 x 28 -> 256, k1 104 -> 84 us.  Not where the gather splits its k * k taps so
+// often that the largest phase's unsplit taps, (k + 1) / 2 squared, make the
+// longer chain (30 x 9 x 9 -> 384, k5 79 -> 131, 128 x 30 x 7 x 7 -> 384, k5 149
+// -> 180 us), nor where the products saved do not pay for the launches added, the
+// filters' and for k = 1 the zeros' (8 x 16 x 64 x 64 -> 24, k3 37 -> 41, 16 x 64
+// x 56 x 56 -> 128, k1 alone 76 -> 88 us).
+DxPlan conv_dx_plan(const ConvGeom& g, bool parts) {
+  DxPlan p{g.s >= 3 || (parts && g.s == 2), {128, 128, 16, 1}, 0};
+  if (g.s == 1 || !p.phased) {
+    p.cfg = dx_choose(g, parts);
+    const uint32_t KK = g.k * g.k, kp = (g.k + 1) / 2;
+    const double products = double(g.C) * g.B * g.H * g.W * KK * pad4(g.OC);
+    p.phased = g.s == 2 && p.cfg.splits * kp * kp <= KK && products >= (g.k == 1 ? 8e8 : 2e8);
+  }
+  if (g.s == 2 && p.phased) p.cfg = dx_choose_phases(g, parts);
+  if (p.cfg.splits > 1) p.part = size_t(p.cfg.splits) * g.C * g.B * g.H * g.W;
+  return p;
+}
+bool conv_dx(const DxPlan& p, const float* w, float* wt, const float* gn, float* dx, float* part,
+             const ConvGeom& g, bool parts) {
+  if (p.phased && g.s == 2) {
+    if (parts) {
+      DxMultiParts r(g, true);
+      return phases_in_one(r, p.cfg, w, wt, gn, dx, part, true);
+    }
+    auto go = [&](auto&& r) { return phases_in_one(r, p.cfg, w, wt, gn, dx, part, false); };
+    return blocked_k(pad4(g.OC)) ? go(DxMulti<true>(g, false)) : go(DxMulti<false>(g, false));
+  }
+  if (p.phased) return dx_phases(w, wt, gn, dx, g, parts);
   if (parts)
-    return g.s == 1
-               ? parts_dispatch(c, DxPartsRun<true, PEpiNCHW>{wt, gn, dx, part, g, c.splits, {}})
-               : parts_dispatch(c, DxPartsRun<false, PEpiNCHW>{wt, gn, dx, part, g, c.splits, {}});
-  return conv_variant<DxRun>(g.s == 1, blocked_k(pad4(g.OC)), c, wt, gn, dx, part, g, c.splits);
+    return g.s == 1 ? parts_dispatch(
+                          p.cfg, DxPartsRun<true, PEpiNCHW>{wt, gn, dx, part, g, p.cfg.splits, {}})
+                    : parts_dispatch(p.cfg, DxPartsRun<false, PEpiNCHW>{wt, gn, dx, part, g,
+                                                                        p.cfg.splits, {}});
+  return conv_variant<DxRun>(g.s == 1, blocked_k(pad4(g.OC)), p.cfg, wt, gn, dx, part, g,
+                             p.cfg.splits);
 }
 
 }  // namespace dce

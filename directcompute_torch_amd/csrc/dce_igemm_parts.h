@@ -525,12 +525,14 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
                                        uint32_t((uint64_t(ktiles) * (z + 1)) / splits));
 }
 
-// Up to four products in one launch, as k_igemm_multi.
+// Up to four products in one launch, as k_igemm_multi; their K in `splits`, the
+// partials `zstride` floats apart.
 template <int MT, int NT, class LA, class LB, class EPI>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
-    k_gemm_parts_multi(const Multi<LA, LB, EPI> a) {
+    k_gemm_parts_multi(const Multi<LA, LB, EPI> a, uint32_t wgs, uint32_t splits,
+                       uint32_t zstride) {
   __shared__ __attribute__((aligned(16))) char S[2 * PTile<MT, NT, LA, LB>::BYTES];
-  const uint32_t id = xcd_block_id();
+  const uint32_t all = xcd_block_id(), z = all / wgs, id = all - z * wgs;
   typename LA::Params pa = a.pa[0];
   typename LB::Params pb = a.pb[0];
   typename EPI::Params pe = a.pe[0];
@@ -544,7 +546,10 @@ __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2
       kt = a.ktiles[i];
       t = id - a.first[i];
     }
-  gemm_parts_tile<MT, NT, LA, LB, EPI>(S, pa, pb, pe, t % a.gm * MT, t / a.gm * NT, 0, 0, kt);
+  pe.out += size_t(z) * zstride;
+  gemm_parts_tile<MT, NT, LA, LB, EPI>(S, pa, pb, pe, t % a.gm * MT, t / a.gm * NT, 0,
+                                       uint32_t((uint64_t(kt) * z) / splits),
+                                       uint32_t((uint64_t(kt) * (z + 1)) / splits));
 }
 
 template <int MT, int NT, class LA, class LB, class EPI>

@@ -34,6 +34,8 @@ CASES = [
     (2, 512, 8, 8, 480, 1, 2, 0, 0),      # k < s: three phases no tap reaches
     (2, 64, 14, 14, 64, 4, 3, 1, 1),      # stride 3: one launch per phase
     (2, 512, 6, 6, 480, 1, 1, 0, 1),      # pointwise with a ReLU mask
+    (7, 137, 6, 7, 505, 3, 2, 0, 0),      # phases of few pixels and long dot products, split
+    (1, 56, 7, 15, 384, 7, 2, 3, 1),      # the same: 16, 12, 12 and 9 taps
 ]
 
 
@@ -238,3 +240,29 @@ def test_forward_alone_pays_nothing(eng):
     held = eng.lib.GetPoolMemory() - before
     assert 4 * B * H * W * 36 <= held < 1.2 * 4 * B * H * W * 36, held
     release(eng, hx, hw, hb, hdy, hy)
+
+
+def _dx_splits(capfd):
+    return [int(l.split("splits ")[1].split()[0]) for l in capfd.readouterr().err.splitlines() if "DCE_TUNE_DX parts" in l]
+
+
+@pytest.mark.parametrize("case", [CASES[14], CASES[15]], ids=str)
+def test_few_pixels_split_the_phases(eng, monkeypatch, capfd, case):
+    """A stride-2 dX whose phases would leave the chip to a few long chains."""
+    monkeypatch.setenv("DCE_TUNE_LOG", "1")
+    x, w, dy, y = _inputs(*case)
+    s, p, act = case[6:]
+    _check(_backward(eng, x, w, dy, y, s, p, act), x, w, dy, y, s, p, act)
+    splits = _dx_splits(capfd)
+    assert len(splits) == 1 and splits[0] > 1, splits
+
+
+@pytest.mark.parametrize("splits", [2, 3, 7])
+def test_split_phases(eng, monkeypatch, splits):
+    """Phases of unequal length (one with fewer steps than splits), odd images, a
+    row without pixels; phases without taps are not split."""
+    monkeypatch.setenv("DCE_TUNE_DX", f"64,128,16,{splits}")
+    for case in CASES[8:12] + [CASES[15]]:
+        x, w, dy, y = _inputs(*case)
+        s, p, act = case[6:]
+        _check(_backward(eng, x, w, dy, y, s, p, act), x, w, dy, y, s, p, act)
