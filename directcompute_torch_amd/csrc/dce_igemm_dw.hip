@@ -78,10 +78,12 @@ struct DwPartsRun {
   ConvGeom g;
   uint32_t splits;
   bool trans;
+  // Layers on parts have at least 200 taps x channels: no 32-row tile of taps.
   template <int MT, int NT>
   int occ(bool) const {
-    return trans ? occupancy(k_gemm_parts<MT, NT, PTap<MT>, PGrad<NT>, PEpiRowMajor>)
-                 : occupancy(k_gemm_parts<MT, NT, PGrad<MT>, PTap<NT>, PEpiRowMajor>);
+    if constexpr (MT > 32)
+      if (trans) return occupancy(k_gemm_parts<MT, NT, PTap<MT>, PGrad<NT>, PEpiRowMajor>);
+    return occupancy(k_gemm_parts<MT, NT, PGrad<MT>, PTap<NT>, PEpiRowMajor>);
   }
   template <int MT, int NT>
   bool run() {
@@ -89,20 +91,25 @@ struct DwPartsRun {
     const uint32_t N = g.k * g.k * nc * 16, zs = 4 * cdiv(size_t(g.OC) * N, 4), kt = cdiv(npix, 16);
     const uint32_t fg = uint32_t(parts_floats(npix, g.OC));
     const uint32_t fx = uint32_t(parts_floats(size_t(g.B) * g.H * g.W, g.C));
+    if (trans) {
+      if constexpr (MT > 32) {
+        const typename PTap<MT>::Params px{xn, g.H, g.W, nc, g.k, g.s, g.p, g.OW, OHW, npix, N, fx,
+                                           make_fastdiv(OHW), make_fastdiv(g.OW),
+                                           make_fastdiv(16 * nc), make_fastdiv(g.k)};
+        const typename PGrad<NT>::Params pg{gn, no, npix, fg};
+        const PEpiRowMajor::Params pe{part, N, g.OC, g.OC, zs};
+        return launch_parts<MT, NT, PTap<MT>, PGrad<NT>, PEpiRowMajor>(px, pg, pe, N, g.OC, kt, splits,
+                                                                       "conv_backward_filter");
+      }
+      set_error("conv_backward_filter: %u taps x channels on a %d-row tile", N, MT);
+      return false;
+    }
     const typename PGrad<MT>::Params pg{gn, no, npix, fg};
-    const typename PTap<MT>::Params px{xn, g.H, g.W, nc, g.k, g.s, g.p, g.OW, OHW, npix, N, fx,
+    const typename PTap<NT>::Params px{xn, g.H, g.W, nc, g.k, g.s, g.p, g.OW, OHW, npix, N, fx,
                                        make_fastdiv(OHW), make_fastdiv(g.OW), make_fastdiv(16 * nc),
                                        make_fastdiv(g.k)};
-    const typename PGrad<NT>::Params pgN{gn, no, npix, fg};
-    const typename PTap<NT>::Params pxN{xn, g.H, g.W, nc, g.k, g.s, g.p, g.OW, OHW, npix, N, fx,
-                                        px.dOHW, px.dOW, px.dC, px.dK};
-    if (trans) {
-      const PEpiRowMajor::Params pe{part, N, g.OC, g.OC, zs};
-      return launch_parts<MT, NT, PTap<MT>, PGrad<NT>, PEpiRowMajor>(px, pgN, pe, N, g.OC, kt, splits,
-                                                                     "conv_backward_filter");
-    }
     const PEpiRowMajor::Params pe{part, g.OC, N, N, zs};
-    return launch_parts<MT, NT, PGrad<MT>, PTap<NT>, PEpiRowMajor>(pg, pxN, pe, g.OC, N, kt, splits,
+    return launch_parts<MT, NT, PGrad<MT>, PTap<NT>, PEpiRowMajor>(pg, px, pe, g.OC, N, kt, splits,
                                                                    "conv_backward_filter");
   }
 };

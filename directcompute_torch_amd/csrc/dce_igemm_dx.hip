@@ -89,8 +89,8 @@ struct DxPhaseRun {
   }
 };
 
-// dX on parts: the whole gather (the phase fields unused), or one phase.
-template <bool S1, class EPI>
+// dX on parts at stride 1 (the phase fields unused), or one phase.
+template <class EPI>
 struct DxPartsRun {
   const float* wt;
   const float* gn;
@@ -102,8 +102,8 @@ struct DxPartsRun {
   static constexpr bool PHASE = std::is_same<EPI, PEpiPhase>::value;
   template <int MT, int NT>
   int occ(bool split) const {
-    return split ? occupancy(k_gemm_parts<MT, NT, PRows<MT>, PPix<NT, S1>, PEpiRowMajor>)
-                 : occupancy(k_gemm_parts<MT, NT, PRows<MT>, PPix<NT, S1>, EPI>);
+    return split ? occupancy(k_gemm_parts<MT, NT, PRows<MT>, PPix<NT>, PEpiRowMajor>)
+                 : occupancy(k_gemm_parts<MT, NT, PRows<MT>, PPix<NT>, EPI>);
   }
   template <int MT, int NT>
   bool run() const {
@@ -112,10 +112,10 @@ struct DxPartsRun {
     const uint32_t kw = PHASE ? q.nw : g.k;
     const char* what = "conv_backward_input";
     using LA = PRows<MT>;
-    using LB = PPix<NT, S1>;
+    using LB = PPix<NT>;
     const typename LA::Params pa{wt, g.C, kt, g.C * kt * 24};
-    const typename LB::Params pb{gn, g.OH, g.OW, no, kw, PHASE ? 1 : g.s, PHASE ? q.qh : g.p, GW, GHW,
-                                 N, uint32_t(parts_floats(size_t(g.B) * g.OH * g.OW, g.OC)),
+    const typename LB::Params pb{gn, g.OH, g.OW, no, kw, PHASE ? q.qh : g.p, GW, GHW, N,
+                                 uint32_t(parts_floats(size_t(g.B) * g.OH * g.OW, g.OC)),
                                  make_fastdiv(GHW), make_fastdiv(GW), make_fastdiv(KK),
                                  make_fastdiv(kw), PHASE ? int(q.qw) - int(q.qh) : 0};
     if constexpr (PHASE) {
@@ -194,24 +194,24 @@ struct DxMultiParts : DxPhases {
   using EPI = PEpiPhase;
   template <int MT, int NT>
   int occ(bool) const {
-    return occupancy(k_gemm_parts_multi<MT, NT, PRows<MT>, PPix<NT, true>, EPI>);
+    return occupancy(k_gemm_parts_multi<MT, NT, PRows<MT>, PPix<NT>, EPI>);
   }
   template <int MT, int NT>
   bool run() const {
-    Multi<PRows<MT>, PPix<NT, true>, EPI> a{};
+    Multi<PRows<MT>, PPix<NT>, EPI> a{};
     const uint32_t no = pad16(g.OC) / 16;
     const uint32_t wgs = fill(a, MT, NT, [&](uint32_t i, const PhaseGeom& f, uint32_t N) {
       const uint32_t KK = f.nh * f.nw, GHW = f.GH * f.GW;
       a.ktiles[i] = KK * no;
       a.pa[i] = {wt[i], g.C, KK * no, g.C * KK * no * 24};
-      a.pb[i] = {gn, g.OH, g.OW, no, f.nw, 1, f.qh, f.GW, GHW, N,
+      a.pb[i] = {gn, g.OH, g.OW, no, f.nw, f.qh, f.GW, GHW, N,
                  uint32_t(parts_floats(size_t(g.B) * g.OH * g.OW, g.OC)), make_fastdiv(GHW),
                  make_fastdiv(f.GW), make_fastdiv(KK), make_fastdiv(f.nw), int(f.qw) - int(f.qh)};
       a.pe[i] = {splits > 1 ? part : dx, g.C,  g.H,  g.W,  f.GW, GHW, N, g.s, f.ph, f.pw,
                  a.pb[i].dGridHW,        a.pb[i].dGridW};
     });
     const uint32_t values = g.B * g.C * g.H * g.W;
-    hipLaunchKernelGGL((k_gemm_parts_multi<MT, NT, PRows<MT>, PPix<NT, true>, EPI>),
+    hipLaunchKernelGGL((k_gemm_parts_multi<MT, NT, PRows<MT>, PPix<NT>, EPI>),
                        dim3(wgs * splits), dim3(kThreads), 0, stream(), a, wgs, splits, values);
     return check_launch("conv_backward_input") &&
            (splits == 1 || split_sum(part, dx, values, splits));
@@ -294,7 +294,7 @@ static bool dx_phases(const float* w, float* wt, const float* gn, float* dx, con
                            q.rw, parts ? 1u : 0u}))
         return false;
       if (parts) {
-        const DxPartsRun<true, PEpiPhase> run{wt, gn, dx, nullptr, g, 1, q};
+        const DxPartsRun<PEpiPhase> run{wt, gn, dx, nullptr, g, 1, q};
         const TileCfg t = parts_choose("DCE_TUNE_DX", g.C, N, kdim, 1, true,
                                        [&](const TileCfg& v) { return parts_occ(v, run); });
         if (!parts_dispatch(t, run)) return false;
@@ -319,12 +319,9 @@ static bool dx_phases(const float* w, float* wt, const float* gn, float* dx, con
 static TileCfg dx_choose(const ConvGeom& g, bool parts) {
   const uint32_t N = g.B * g.H * g.W;
   const bool s1 = g.s == 1;
-  if (parts)
+  if (parts)  // s1: conv_dx_plan takes the phases otherwise
     return parts_choose("DCE_TUNE_DX", g.C, N, g.k * g.k * pad16(g.OC), 8, true,
-                        [&](const TileCfg& t) {
-                          return s1 ? parts_occ(t, DxPartsRun<true, PEpiNCHW>{})
-                                    : parts_occ(t, DxPartsRun<false, PEpiNCHW>{});
-                        });
+                        [&](const TileCfg& t) { return parts_occ(t, DxPartsRun<PEpiNCHW>{}); });
   const uint32_t OCp = pad4(g.OC), kdim = g.k * g.k * OCp;
   const bool blk = blocked_k(OCp);
   TileCfg c = choose(
@@ -390,11 +387,13 @@ bool conv_dx(const DxPlan& p, const float* w, float* wt, const float* gn, float*
     return blocked_k(pad4(g.OC)) ? go(DxMulti<true>(g, false)) : go(DxMulti<false>(g, false));
   }
   if (p.phased) return dx_phases(w, wt, gn, dx, g, parts);
-  if (parts)
-    return g.s == 1 ? parts_dispatch(
-                          p.cfg, DxPartsRun<true, PEpiNCHW>{wt, gn, dx, part, g, p.cfg.splits, {}})
-                    : parts_dispatch(p.cfg, DxPartsRun<false, PEpiNCHW>{wt, gn, dx, part, g,
-                                                                        p.cfg.splits, {}});
+  if (parts) {
+    if (g.s != 1) {
+      set_error("conv_backward_input: a strided gather has no kernel on parts");
+      return false;
+    }
+    return parts_dispatch(p.cfg, DxPartsRun<PEpiNCHW>{wt, gn, dx, part, g, p.cfg.splits, {}});
+  }
   return conv_variant<DxRun>(g.s == 1, blocked_k(pad4(g.OC)), p.cfg, wt, gn, dx, part, g,
                              p.cfg.splits);
 }

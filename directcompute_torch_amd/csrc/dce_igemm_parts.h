@@ -76,7 +76,7 @@ constexpr uint32_t kOobBytes = kOob * 4u;
 // ---------------------------------------------------------------------------
 template <int R, bool KROW>
 struct PStage {
-  static_assert(R == 32 || R == 64 || R == 128 || R == 256, "rows of a tile");
+  static_assert(R == 32 || R == 64 || R == 128, "rows of a tile");
   static constexpr int QP = 2 * R;  // quads per part
   static constexpr int LOADS = (3 * QP + kThreads - 1) / kThreads;
   static constexpr int BYTES = 3 * QP * 16;
@@ -179,21 +179,21 @@ struct PRows : PLoader<R, false> {
   }
 };
 
-// G patches for dX: rows = input pixels, K tile kt = (channel block, tap);
-// LdPixRK's blocked order.
-template <int R, bool S1>
+// G patches for dX at stride 1 (a layer, or a sub-pixel phase): rows = input
+// pixels, K tile kt = (channel block, tap); LdPixRK's blocked order.
+template <int R>
 struct PPix : PLoader<R, false> {
   using St = PStage<R, false>;
   static constexpr bool KROW = false;
   struct Params {
     const float* src;
-    uint32_t srcH, srcW, nblk, k, s, p, gridW, gridHW, N, n;
+    uint32_t srcH, srcW, nblk, k, p, gridW, gridHW, N, n;
     FastDiv dGridHW, dGridW, dKK, dK;
     int pwd;  // the column origin is c + p + pwd
   };
-  uint32_t srcH, srcW, nblk, k, s;
+  uint32_t srcH, srcW, nblk, k;
   FastDiv dKK, dK;
-  uint32_t pbase[St::UN], qbase[St::UN];
+  uint32_t qbase[St::UN];
   int r0[St::UN], c0[St::UN];
   __device__ __forceinline__ void init(const Params& P, uint32_t row0, int t) {
     this->base_init(P.src, P.n, t);
@@ -201,7 +201,6 @@ struct PPix : PLoader<R, false> {
     srcW = P.srcW;
     nblk = P.nblk;
     k = P.k;
-    s = P.s;
     dKK = P.dKK;
     dK = P.dK;
 #pragma unroll
@@ -209,29 +208,20 @@ struct PPix : PLoader<R, false> {
       const uint32_t n = row0 + St::row(t, u);
       const uint32_t bb = fdiv(n, P.dGridHW), rem = n - bb * P.gridHW;
       const uint32_t a = fdiv(rem, P.dGridW), c = rem - a * P.gridW;
-      pbase[u] = bb * P.srcH * P.srcW;
       r0[u] = n < P.N ? int(a + P.p) : (1 << 20);  // past the grid: no tap is in the image
       c0[u] = int(c + P.p) + P.pwd;
       // Offset of tap (0, 0), modulo 2^32 (the origin may lie in the padding).
-      qbase[u] = (pbase[u] + uint32_t(r0[u]) * P.srcW + uint32_t(c0[u])) * P.nblk * kBlkBytes +
+      qbase[u] = (bb * P.srcH * P.srcW + uint32_t(r0[u]) * P.srcW + uint32_t(c0[u])) * P.nblk *
+                     kBlkBytes +
                  St::byte(t, u);
     }
   }
   __device__ __forceinline__ uint32_t off(uint32_t kt, int u) const {
     const uint32_t cb = fdiv(kt, dKK), khw = kt - cb * dKK.d;
     const uint32_t kh = fdiv(khw, dK), kw = khw - kh * k;
-    bool ok = cb < nblk;
-    int h = r0[u] - int(kh), w = c0[u] - int(kw);
-    if constexpr (S1) {
-      ok = ok && uint32_t(h) < srcH && uint32_t(w) < srcW;
-      return ok ? qbase[u] + (cb * kBlkBytes - (kh * srcW + kw) * nblk * kBlkBytes) : kOobBytes;
-    }
-    ok = ok && h >= 0 && w >= 0;
-    const uint32_t oh = uint32_t(h) / s, ow = uint32_t(w) / s;
-    ok = ok && oh * s == uint32_t(h) && ow * s == uint32_t(w) && oh < srcH && ow < srcW;
-    return ok ? ((pbase[u] + oh * srcW + ow) * nblk + cb) * kBlkBytes +
-                    St::byte(this->tid, u)
-              : kOobBytes;
+    const int h = r0[u] - int(kh), w = c0[u] - int(kw);
+    const bool ok = cb < nblk && uint32_t(h) < srcH && uint32_t(w) < srcW;
+    return ok ? qbase[u] + (cb * kBlkBytes - (kh * srcW + kw) * nblk * kBlkBytes) : kOobBytes;
   }
 };
 
