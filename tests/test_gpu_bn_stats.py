@@ -253,6 +253,9 @@ BNG_CASES = [
     (1, 8, 9, 9, 6, 5, 1, 2),         # OC not a multiple of 4 (padded G rows)
     (2, 24, 10, 10, 40, 3, 2, 1),     # stride 2 (the forward leaves no statistics: plain BN dx)
     (2, 24, 8, 8, 36, 1, 1, 0),       # pointwise: no transpose pass, plain BN dx
+    (2, 64, 13, 17, 72, 3, 1, 1),     # G as bf16 parts: five blocks of 16, the last half full
+    (2, 33, 9, 7, 129, 3, 1, 1),      # nine blocks, the last of one channel
+    (1, 96, 11, 9, 32, 3, 1, 1),      # two blocks: the 32-row tile's dW
 ]
 
 

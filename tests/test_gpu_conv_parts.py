@@ -102,6 +102,23 @@ def test_forced_tiles(eng, monkeypatch, tile):
         _check(_backward(eng, x, w, dy, y, s, p, act), x, w, dy, y, s, p, act)
 
 
+@pytest.mark.parametrize("splits", [1, 2, 5])
+@pytest.mark.parametrize("case,var", [
+    ((1, 96, 11, 13, 32, 3, 1, 1, 1), "DCE_TUNE_DW"),   # 32 output channels
+    ((2, 90, 9, 7, 32, 5, 2, 2, 0), "DCE_TUNE_DW"),
+    ((1, 32, 7, 9, 384, 5, 1, 2, 0), "DCE_TUNE_DX"),    # 32 input channels, ragged pixels
+    ((2, 32, 11, 10, 300, 3, 2, 1, 1), "DCE_TUNE_DX"),  # their phases
+], ids=str)
+def test_32_row_tiles(eng, monkeypatch, capfd, case, var, splits):
+    monkeypatch.setenv(var, f"32,128,16,{splits}")
+    monkeypatch.setenv("DCE_TUNE_LOG", "1")
+    x, w, dy, y = _inputs(*case)
+    s, p, act = case[6:]
+    _check(_backward(eng, x, w, dy, y, s, p, act), x, w, dy, y, s, p, act)
+    log = [l for l in capfd.readouterr().err.splitlines() if f"{var} parts" in l]
+    assert log and all("-> 32x128" in l for l in log), log
+
+
 @pytest.mark.parametrize("what", ["inf", "nan", "quiet", "overflow", "tiny", "tiny weights", "few tiny", "denormal"])
 def test_special_values(eng, what):
     """Infinities and NaNs come out where IEEE arithmetic puts them (the tile is
