@@ -363,14 +363,20 @@ static TileCfg dx_choose_phases(const ConvGeom& g, bool parts) {
 // longer chain (30 x 9 x 9 -> 384, k5 79 -> 131, 128 x 30 x 7 x 7 -> 384, k5 149
 // -> 180 us), nor where the products saved do not pay for the launches added, the
 // filters' and for k = 1 the zeros' (8 x 16 x 64 x 64 -> 24, k3 37 -> 41, 16 x 64
-// x 56 x 56 -> 128, k1 alone 76 -> 88 us).
+// x 56 x 56 -> 128, k1 alone 76 -> 88 us), nor under short dot products, where
+// the phases' stores, every second float of a row, bound them (48 x 390 x 118 x
+// 16 -> 4, k2 163 -> 226, 67 x 55 x 182 x 67 -> 6, k3 319 -> 384, 27 x 220 x 49 x
+// 35 -> 9, k3 99 -> 110; but 83 x 20 x 137 x 68 -> 48, k2 229 -> 196, 6 x 10 x 129
+// x 146 -> 21, k3 52 -> 49 and, over few channels, 112 x 9 x 26 x 145 -> 9, k3 70
+// -> 64 us).
 DxPlan conv_dx_plan(const ConvGeom& g, bool parts) {
   DxPlan p{g.s >= 3 || (parts && g.s == 2), {128, 128, 16, 1}, 0};
   if (g.s == 1 || !p.phased) {
     p.cfg = dx_choose(g, parts);
     const uint32_t KK = g.k * g.k, kp = (g.k + 1) / 2;
     const double products = double(g.C) * g.B * g.H * g.W * KK * pad4(g.OC);
-    p.phased = g.s == 2 && p.cfg.splits * kp * kp <= KK && products >= (g.k == 1 ? 8e8 : 2e8);
+    p.phased = g.s == 2 && p.cfg.splits * kp * kp <= KK && products >= (g.k == 1 ? 8e8 : 2e8) &&
+               KK * pad4(g.OC) >= (g.C > 16 ? 180u : 100u);
   }
   if (g.s == 2 && p.phased) p.cfg = dx_choose_phases(g, parts);
   if (p.cfg.splits > 1) p.part = size_t(p.cfg.splits) * g.C * g.B * g.H * g.W;

@@ -63,3 +63,16 @@ def test_dx_phases(eng, case):
         worst = np.max(np.abs(got - ref) - (OC * k * k + 2) * 2.0 ** -24 * S)
         assert worst <= 1e-37, f"{worst:.3e} past the bound"
     release(eng, *hs, hy)
+
+
+@pytest.mark.parametrize("case,phased", [
+    ((16, 100, 63, 64, 8, 2, 0, 0), False),   # dot products of 32: the gather
+    ((10, 60, 64, 63, 9, 4, 1, 0), True),     # 192
+    ((60, 9, 64, 65, 9, 3, 1, 0), True),      # 108, over few channels
+], ids=str)
+def test_short_dot_products_gather(eng, monkeypatch, capfd, case, phased):
+    """The choice logs one tile for the gather and a second one for the phases."""
+    monkeypatch.setenv("DCE_TUNE_LOG", "1")
+    test_dx_phases(eng, case)
+    lines = [l for l in capfd.readouterr().err.splitlines() if "DCE_TUNE_DX" in l]
+    assert len(lines) == 2 * (1 + phased), lines  # two calls
