@@ -425,7 +425,7 @@ struct LdNchwRK : LoaderBase<Stage<R, KT, false>> {
 //        oh*s == a + p - kh exactly (S1: s == 1, no divisibility test).
 //        A strided dX runs as s*s sub-pixel phases, each an S1 gather over
 //        its own grid of input pixels with nh x nw taps (k = nw) and the
-//        column origin shifted by pwd (conv_dx_plan).
+//        column origin shifted by pwd (dx_phase_params).
 // ---------------------------------------------------------------------------
 constexpr int kCB = 16;
 
@@ -1543,7 +1543,7 @@ struct WPerm {
   int mode, blocked;
   uint32_t vw, kk, s, rh, rw;
   // Blocked order with inner % 16 == 0: out as bf16 parts, 96 bytes per
-  // block of 16 k (split_parts).
+  // block of 16 k (split_pair).
   uint32_t parts;
   uint32_t blocks() const { return w ? cdiv(size_t(mode == 0 ? OC : C) * ld, 256) : 0; }
 };

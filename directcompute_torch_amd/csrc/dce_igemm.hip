@@ -927,11 +927,11 @@ bool pw_x(const ConvGeom& g) {
 bool packed_x(const ConvGeom& g) { return g.C < 4 && g.s > 4; }
 // Does the backward run on bf16 parts (dce_igemm_parts.h)?  The parts cost
 // traffic (the forward's copy of x split to 6 bytes a value, G written and read
-// as 6 instead of 4), which C * OC * k * k products per pixel
-// have to pay for: 3 x 3 layers over 32 -> 32 and 32 -> 64 channels lose
-// (forward, passes and backward 136 -> 150 us at 8 x 128 x 128, 94 -> 108 us
-// at 8 x 64 x 64), 96 -> 32 and 64 -> 64 gain (303 -> 284, 133 -> 128 us), 384
-// -> 256 at 13 x 13, b128: 978 -> 824 us.
+// as 6 instead of 4), which C * OC * k * k products per pixel have to pay for:
+// 3 x 3 layers over 32 -> 32 and 32 -> 64 channels lose (forward and backward on
+// fp32 and on parts 111 and 114 us at 8 x 128 x 128, 70 and 73 at 8 x 64 x 64),
+// 96 -> 32 and 64 -> 64 gain (246 and 228, 104 and 94 us), 384 -> 256 at 13 x
+// 13, b128: 942 and 714 us.
 bool conv_parts(const ConvGeom& g) {
   if (g.C < 32 || g.OC < 32) return false;
   // dW over less than one 16-deep step gains nothing, and a sum of one product is

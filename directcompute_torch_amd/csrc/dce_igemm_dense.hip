@@ -43,8 +43,8 @@ struct GemmRun {
 // the fp32 MFMAs, at twice the time that reading W takes; as in the
 // convolutions' backward, six bf16 products stand for one fp32 product.  W is
 // read once by each row of tiles, so both operands are split on their way from
-// registers into LDS.  128 x 4096 x 9216: 97 -> 73 us; 512 x 4096 x 9216: 361 -> 281 us;
-// error against float64 4.4e-7 -> 1.9e-7 and 6.6e-7 -> 2.5e-7.
+// registers into LDS.  128 x 4096 x 9216: 90 -> 74 us; 512 x 4096 x 9216: 355 -> 269 us;
+// error against float64 4.4e-7 -> 1.5e-7 (over 2048: 2.9e-7 -> 1.2e-7).
 //
 // Not taken for A^T B (the filter gradient: both operands split by a pass
 // 107 -> 106 us at 9216 x 128 x 4096, 46 -> 56 us at 4096 x 128 x 4096; its
@@ -213,9 +213,9 @@ static int dense_occ(const TileCfg& c, const F& f) {
   return 1;
 }
 
-// More than one 64-row tile and at least 2e9 products: 96 x 4096 x 4096 44 ->
-// 40, 200 x 4096 x 4096 86 -> 66, 320 x 9000 x 700 (rows x columns x K) 58 ->
-// 41, 512 x 1500 x 4096 66 -> 55 us; 256 x 2048 x 2048 (33 -> 34) and 200 x 700
+// More than one 64-row tile and at least 2e9 products: 96 x 4096 x 4096 41 and
+// 41, 200 x 4096 x 4096 85 -> 64, 320 x 9000 x 700 (rows x columns x K) 57 ->
+// 43, 512 x 1500 x 4096 64 -> 53 us; 256 x 2048 x 2048 (33 -> 34) and 200 x 700
 // x 900 (12.5 -> 14.4 us) stay on fp32 MFMAs.  Over many rows the dot products
 // have to be long as well: 500 x 4000 x 1200 loses (54 -> 59 us).
 static bool dense_on_parts(uint32_t M, uint32_t K, uint32_t N, bool aT, bool bT) {

@@ -33,8 +33,9 @@
 // bytes).  Split inside the GEMM instead, each element is split again for
 // every tile that reads it, and the vector unit bounds the kernel: with the
 // split after the LDS read 8.1 vector instructions per MFMA and the matrix
-// unit 37 % busy (64 -> 128 channels, 56 x 56: dW 433 us), with the split
-// before the LDS write and one LDS stage 476 us, with fp32 MFMAs 495 us.
+// unit 37 % busy (64 -> 128 channels, 56 x 56, b128: dW 433 us), with the split
+// before the LDS write and one LDS stage 476 us, with fp32 MFMAs 495 us, split
+// once and kept 343 us (matrix unit 50 % busy, address unit 73 %).
 //
 // An operand without three bf16 parts (infinite, NaN, so large that it rounds to
 // infinity, or not zero and below 2^-110 = 8e-34) is kept as a NaN and its own
@@ -559,10 +560,11 @@ static bool launch_parts(const typename LA::Params& pa, const typename LB::Param
 // n in batches of at most the kernel's occupancy; a step (16 k) of a batch of r
 // takes lat + r * step, fitted per tile to sweeps of the AlexNet and UNet
 // layers and the 64 -> 128 channel 56 x 56 one: 128 x 128 takes 0.95 us alone
-// on its CU and 1.40 us in pairs (188 TFLOP/s), 64 x 128 0.8 us in pairs and
-// 1.4 us in fours, the small tiles 0.65 - 0.8 us up to three at a time.  At 200
-// TFLOP/s this card's bf16 matrix products are at their power limit (8192^3:
-// 1.2 PFLOP/s).
+// on its CU and 1.40 us in pairs, 64 x 128 0.8 us in pairs and 1.4 us in fours,
+// the small tiles 0.65 - 0.8 us up to three at a time.  The fits are from
+// kernels that added the small products to the accumulator after every step;
+// without those adds every tile is some 5 % faster, and the AlexNet layers
+// reach 172 - 260 TFLOP/s with the choices made.
 struct PartsTile {
   int MT, NT;
   double lat, step;
