@@ -119,7 +119,7 @@ def test_32_row_tiles(eng, monkeypatch, capfd, case, var, splits):
     assert log and all("-> 32x128" in l for l in log), log
 
 
-@pytest.mark.parametrize("what", ["inf", "nan", "quiet", "overflow", "tiny", "tiny weights", "few tiny", "denormal"])
+@pytest.mark.parametrize("what", ["inf", "nan", "quiet", "overflow", "tiny", "tiny weights", "few tiny", "denormal", "largest"])
 def test_special_values(eng, what):
     """Infinities and NaNs come out where IEEE arithmetic puts them (the tile is
     computed again in fp32), and so do values below the range of three bf16 parts,
@@ -143,6 +143,9 @@ def test_special_values(eng, what):
         x[:, 9] *= np.float32(2e-37)
         w[:, 9] *= np.float32(2e-37)
         dy[:, 70] *= np.float32(2e-37)
+    elif what == "largest":  # finite, but rounds to infinity as bf16; its products stay finite
+        dy[1, 60, 4, 4] = np.finfo(np.float32).max
+        x, w = x * np.float32(1e-3), w * np.float32(1e-3)
     else:
         dy *= np.float32(1e-39)
     with np.errstate(all="ignore"):
@@ -158,7 +161,7 @@ def test_special_values(eng, what):
         fin = np.isfinite(b32)
         scale = np.max(np.abs(b[fin])) if what != "overflow" else np.maximum(np.abs(b[fin]), 1.0)
         tol = 1e-5
-        if "tiny" in what or what == "denormal":
+        if "tiny" in what or what in ("denormal", "largest"):
             Sm = K.conv_backward(np.abs(dy), y, np.abs(x), np.abs(w), s, p, act)
             Sm, n = (Sm[0], 180) if a is got[0] else (Sm[2], 720)
             assert np.all(np.abs(a - b) <= (n + 256) * (2.0 ** -24 * Sm + 2.0 ** -149))

@@ -89,6 +89,19 @@ def test_a_bt_error_and_bias_against_fp32_fmas(eng, monkeypatch, terms):
     assert abs(err.mean()) <= 2.0 ** -28 + terms * 2.0 ** -38
 
 
+def test_a_bt_largest(eng):
+    """Finite values that round to infinity as bf16, with finite products."""
+    M, Kd, N = 130, 4100, 3800
+    r = rng(23)
+    a = r.standard_normal((M, Kd), dtype=np.float32)
+    b = r.standard_normal((N, Kd), dtype=np.float32) * np.float32(1e-3)
+    a[7, 4099], a[129, 0] = np.finfo(np.float32).max, np.float32(-3.3999e38)
+    ref = a.astype(np.float64) @ b.T.astype(np.float64)
+    S = np.abs(a).astype(np.float64) @ np.abs(b).T.astype(np.float64)
+    c = _matmul(eng, a, b)
+    assert np.all(np.isfinite(c)) and np.all(np.abs(c - ref) <= 64 * 2.0 ** -24 * S)
+
+
 @pytest.mark.parametrize("scale", [1e-36, 1e-39, 1e-33])
 @pytest.mark.parametrize("which", ["a", "b", "row"])
 def test_a_bt_tiny(eng, which, scale):
